@@ -91,10 +91,23 @@ struct PivotFront
 };
 
 // Where a front's Bunch–Kaufman elimination stands: the next position k, the end of the candidates still to try in
-// this pass, the start of the pass, done (1: e = k), and the 2 × 2 blocks taken.
+// this pass, the start of the pass, done (1: e = k), the 2 × 2 blocks taken, and the first column of the last step
+// (its trailing update takes the columns [from, k)).
 struct PivotState
 {
-    int32_t k, end, passStart, done, twoByTwo, pad0, pad1, pad2;
+    int32_t k, end, passStart, done, twoByTwo, from, pad0, pad1;
+};
+
+// The steps of the Bunch–Kaufman elimination: up to PIVOT_PANEL columns each, by the rows from the step's first column
+// on (launchPivotStep's kind): in the registers of 256 threads, of 512 threads, or (any number) in memory.
+constexpr int PIVOT_PANEL = 16;
+constexpr int PIVOT_SMALL_ROWS = 512, PIVOT_LARGE_ROWS = 4096;
+enum
+{
+    PIVOT_SMALL = 0,
+    PIVOT_LARGE,
+    PIVOT_ANY,
+    PIVOT_KINDS
 };
 
 // Columns [j0, j1) of a child's update matrix (M × M at src, leading dimension lds) added into its parent's front
@@ -300,8 +313,12 @@ hipError_t launchScaleRows(const double* src, double* dst, const double* scale, 
 hipError_t launchAddRows(double* x, const double* z, int64_t n, int k, hipStream_t stream);
 hipError_t launchPlainUpdateTiles(double* fronts, const double* w, const UpdateTile* tiles, int count,
                                   hipStream_t stream);
-hipError_t launchBunchKaufman(const PivotFront* fronts, PivotState* states, const int32_t* list, int count, int nb,
-                              hipStream_t stream);
+// One step of each front of the list (fronts of the rows that `kind` holds), then its trailing update on the items
+// {front, row tile, column tile} of 64 × 64.
+hipError_t launchPivotStep(int kind, const PivotFront* fronts, PivotState* states, const int32_t* list, int count,
+                           hipStream_t stream);
+hipError_t launchPivotTrailing(const PivotFront* fronts, const PivotState* states, const int4* items, int count,
+                               hipStream_t stream);
 hipError_t launchPivotMatrix(const DeviceMatrix& a, const PivotFront* fronts, int count, hipStream_t stream);
 hipError_t launchPivotExtendAdd(const ExtendItem* items, int count, hipStream_t stream);
 hipError_t launchCopyRanges(const CopyRange* ranges, int count, hipStream_t stream);

@@ -2488,52 +2488,108 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                                                  rankStart[rank + 1] - rankStart[rank], st),
                       "factor: extend-add");
         }
-        // Block steps until every front of the level is done, each followed by its trailing tiles.
-        std::vector<int32_t> active(count), next;
+        // Steps until every front of the level is done, each followed by its trailing update, in rounds: a round
+        // launches for each front the steps its candidates need and a few more (a column that interchanges ends its
+        // step early), with no wait between them (the launches read the fronts' states on the device, and a front that
+        // is done does nothing), then reads the states. The fronts that need most steps come first, so that every
+        // launch of a round takes the first ones of its list.
+        std::vector<oosg::UpdateTile> tiles;
+        std::vector<int32_t> active(count), list32;
         for (int q = 0; q < count; ++q)
             active[q] = q;
-        std::vector<int32_t> kNow(count, 0);
-        std::vector<oosg::UpdateTile> tiles;
-        // Every step of a front eliminates PANEL_BLOCK columns or ends a pass, and a pass that eliminates nothing
-        // ends the front: this bounds the steps.
+        std::vector<int4> trailing;
+        // Every step of a front eliminates a column or ends a pass, and a pass that eliminates nothing ends the
+        // front: this bounds the rounds.
         int32_t maxCand = 0;
         for (int q = 0; q < count; ++q)
             maxCand = std::max(maxCand, cand[list[q]]);
-        int64_t stepsLeft = 2 * int64_t(maxCand) + 8;
+        int64_t roundsLeft = 2 * int64_t(maxCand) + 8;
         while (!active.empty())
         {
-            if (--stepsLeft < 0)
+            const auto rowsOf = [&](int32_t q) { return pf->order[list[q]] - states[q].k; };
+            const auto kindOf = [&](int32_t q)
+            {
+                const int rows = rowsOf(q);
+                return rows <= oosg::PIVOT_SMALL_ROWS   ? oosg::PIVOT_SMALL
+                       : rows <= oosg::PIVOT_LARGE_ROWS ? oosg::PIVOT_LARGE
+                                                        : oosg::PIVOT_ANY;
+            };
+            const auto stepsOf = [&](int32_t q)
+            {
+                // Panels of half the width where the rows need most registers (eliminatePanel).
+                const int width = oosg::PIVOT_PANEL / (rowsOf(q) > oosg::PIVOT_LARGE_ROWS / 2 ? 2 : 1);
+                const int steps = (cand[list[q]] - states[q].k + width - 1) / width;
+                return steps + steps / 32 + 1;
+            };
+            std::sort(active.begin(), active.end(),
+                      [&](int32_t x, int32_t y)
+                      {
+                          const int sx = stepsOf(x), sy = stepsOf(y);
+                          return sx != sy ? sx > sy : x < y;
+                      });
+            list32.clear();
+            trailing.clear();
+            std::vector<int> kindStart(oosg::PIVOT_KINDS + 1, 0);
+            std::vector<std::vector<int>> kindSteps(oosg::PIVOT_KINDS);
+            for (int kind = 0; kind < oosg::PIVOT_KINDS; ++kind)
+            {
+                for (const int32_t q : active)
+                    if (kindOf(q) == kind)
+                    {
+                        list32.push_back(q);
+                        kindSteps[kind].push_back(stepsOf(q));
+                    }
+                kindStart[kind + 1] = static_cast<int>(list32.size());
+            }
+            std::vector<int> tileSteps, tileEnd; // per active front: its steps, the end of its tiles
+            for (const int32_t q : active)
+            {
+                const int C = cand[list[q]], N = pf->order[list[q]];
+                for (int J = states[q].k / 64; 64 * J < C; ++J)
+                    for (int I = J; 64 * I < N; ++I)
+                        trailing.push_back(make_int4(q, I, J, 0));
+                tileSteps.push_back(stepsOf(q));
+                tileEnd.push_back(static_cast<int>(trailing.size()));
+            }
+            uploadInto(p.pivotList, list32, st, "factor: active fronts");
+            uploadInto(p.pivotTiles, trailing, st, "factor: trailing tiles");
+            const int steps = tileSteps.front();
+            if (--roundsLeft < 0)
                 fail(OOSG_INTERNAL, "factor: the Bunch-Kaufman steps of a level did not end");
-            uploadInto(p.pivotList, active, st, "factor: active fronts");
-            check(oosg::launchBunchKaufman(desc, dStates, p.pivotList.as<int32_t>(), static_cast<int>(active.size()),
-                                           oosg::PANEL_BLOCK, st),
-                  "factor: Bunch-Kaufman");
+            size_t taking = active.size();
+            for (int step = 0; step < steps; ++step)
+            {
+                for (int kind = 0; kind < oosg::PIVOT_KINDS; ++kind)
+                {
+                    std::vector<int>& left = kindSteps[kind];
+                    while (!left.empty() && left.back() <= step)
+                        left.pop_back();
+                    check(oosg::launchPivotStep(kind, desc, dStates, p.pivotList.as<int32_t>() + kindStart[kind],
+                                                static_cast<int>(left.size()), st),
+                          "factor: Bunch-Kaufman");
+                }
+                while (taking > 0 && tileSteps[taking - 1] <= step)
+                    --taking;
+                check(oosg::launchPivotTrailing(desc, dStates, p.pivotTiles.as<int4>(),
+                                                taking > 0 ? tileEnd[taking - 1] : 0, st),
+                      "factor: trailing update");
+            }
+            std::vector<int32_t> kBefore(static_cast<size_t>(count));
+            for (int q = 0; q < count; ++q)
+                kBefore[q] = states[q].k;
             check(hipMemcpyAsync(states.data(), dStates, states.size() * sizeof(oosg::PivotState),
                                  hipMemcpyDeviceToHost, st),
                   "factor: front states");
             check(hipStreamSynchronize(st), "factor: Bunch-Kaufman");
-            tiles.clear();
-            next.clear();
+            size_t kept = 0;
             for (const int32_t q : active)
             {
-                const int32_t s = list[q];
-                const int kb = kNow[q], ka = states[q].k;
-                if (ka < kb || ka > cand[s])
+                if (states[q].k < kBefore[q] || states[q].k > cand[list[q]])
                     fail(OOSG_INTERNAL, "factor: a front's elimination went back");
-                if (ka > kb)
-                    addPivotTiles(tiles, fOff[q], wOff[q], pf->order[s], ka, cand[s], kb, ka);
-                kNow[q] = ka;
                 if (!states[q].done)
-                    next.push_back(q);
+                    active[kept++] = q;
             }
-            if (!tiles.empty())
-            {
-                uploadInto(p.pivotTiles, tiles, st, "factor: trailing tiles");
-                check(oosg::launchPlainUpdateTiles(F0, W0, p.pivotTiles.as<oosg::UpdateTile>(),
-                                                   static_cast<int>(tiles.size()), st),
-                      "factor: trailing tiles");
-            }
-            active.swap(next);
+            active.resize(kept);
         }
         // The rows below the candidates: their update matrix part −= L·Wᵀ over the eliminated columns.
         tiles.clear();

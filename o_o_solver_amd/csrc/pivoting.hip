@@ -3,10 +3,12 @@
 //
 // A pivoted front is a full N × N column-major array (leading dimension N, lower triangle used) whose positions are
 // [the supernode's own c columns, the d columns its children delayed, its r rows]; the first C = c + d are the
-// candidates. Its elimination runs in blocks of columns on one workgroup per front (bunchKaufmanKernel), each column
-// computed left-looking from the block's columns (W = the updated columns, L·D), then the columns of the candidates
-// to the right get C −= L·Wᵀ by MFMA tiles (updateTilesKernel<double, true>) and, after the last block, the rows
-// below the candidates likewise with K = e (the eliminated count). The pivot tests are those of
+// candidates. Its elimination runs in steps of up to 16 columns: one workgroup per front eliminates them
+// (pivotPanelKernel, the rows in registers; pivotColumnsKernel for fronts with more rows than those hold), W = the
+// updated columns, L·D; then the candidates to the right get C −= L·Wᵀ by MFMA tiles that read from the front's state
+// how far the step got (pivotTrailingKernel), so the host launches a level's steps without waiting for each. After
+// the last step the rows below the candidates get the same product with K = e, the eliminated count
+// (updateTilesKernel<double, true>). The pivot tests are those of
 // src/linalg/kernels/reference/DenseBlockKernels.cpp:448-580: α = (1 + √17)/8, and a candidate whose partner row is
 // not a candidate is pivoted alone when |a_kk| >= 0.01·colmax and delayed otherwise (moved behind the candidates still
 // to try); passes over the delayed candidates repeat while a pass eliminates something.
@@ -19,6 +21,8 @@
 
 namespace oosg
 {
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
 
 namespace
 {
@@ -89,16 +93,17 @@ __device__ inline void updatedColumn(const double* F, double* W, int N, int k0, 
 // The symmetric interchange of positions p < q of the front (DenseBlockKernels.cpp:69-79), over the stored values:
 // rows p and q of the columns before p (the eliminated columns' L, and the columns still to come), the parts between,
 // below and on the diagonal; with rows p and q of the block's W columns and the permutation.
+template <int THREADS>
 __device__ inline void interchange(double* F, double* W, int32_t* perm, int N, int k0, int k, int p, int q)
 {
     const int tid = threadIdx.x;
-    for (int t = tid; t < p; t += BK_THREADS)
+    for (int t = tid; t < p; t += THREADS)
         swapValues(F[p + int64_t(t) * N], F[q + int64_t(t) * N]);
-    for (int i = p + 1 + tid; i < q; i += BK_THREADS)
+    for (int i = p + 1 + tid; i < q; i += THREADS)
         swapValues(F[i + int64_t(p) * N], F[q + int64_t(i) * N]);
-    for (int i = q + 1 + tid; i < N; i += BK_THREADS)
+    for (int i = q + 1 + tid; i < N; i += THREADS)
         swapValues(F[i + int64_t(p) * N], F[i + int64_t(q) * N]);
-    for (int t = k0 + tid; t < k; t += BK_THREADS)
+    for (int t = k0 + tid; t < k; t += THREADS)
         swapValues(W[p + int64_t(t) * N], W[q + int64_t(t) * N]);
     if (tid == 0)
     {
@@ -110,10 +115,11 @@ __device__ inline void interchange(double* F, double* W, int32_t* perm, int N, i
     __syncthreads();
 }
 
-// One block step of the Bunch–Kaufman elimination of each front of the list (one workgroup per front): from the
-// front's state, columns are eliminated until `nb` of them are (one more when the last pivot is 2 × 2) or the
-// candidates are done. The state records where the next step starts.
-__global__ __launch_bounds__(BK_THREADS) void bunchKaufmanKernel(const PivotFront* fronts, PivotState* states,
+// One step of the Bunch–Kaufman elimination of each front of the list (one workgroup per front), for fronts of any
+// size: from the front's state, columns are eliminated until `nb` of them are (one more when the last pivot is 2 × 2)
+// or the candidates are done, each column computed left-looking from the step's columns in memory. The state records
+// where the step started and where the next one does.
+__global__ __launch_bounds__(BK_THREADS) void pivotColumnsKernel(const PivotFront* fronts, PivotState* states,
                                                                  const int32_t* list, int nb)
 {
     __shared__ double wr[2 * PANEL_BLOCK + 8];
@@ -123,7 +129,11 @@ __global__ __launch_bounds__(BK_THREADS) void bunchKaufmanKernel(const PivotFron
     const PivotFront fr = fronts[q];
     const PivotState st = states[q];
     if (st.done)
+    {
+        if (threadIdx.x == 0)
+            states[q].from = st.k;
         return;
+    }
     double* F = fr.F;
     double* W = fr.W;
     int32_t* perm = fr.perm;
@@ -180,7 +190,7 @@ __global__ __launch_bounds__(BK_THREADS) void bunchKaufmanKernel(const PivotFron
                 // The partner is not a candidate and the diagonal is too small: delay the column.
                 --end;
                 if (k != end)
-                    interchange(F, W, perm, N, k0, k, k, end);
+                    interchange<BK_THREADS>(F, W, perm, N, k0, k, k, end);
                 continue;
             }
         }
@@ -206,7 +216,7 @@ __global__ __launch_bounds__(BK_THREADS) void bunchKaufmanKernel(const PivotFron
         const int moved = k + blockSize - 1;
         if (swapWith != moved)
         {
-            interchange(F, W, perm, N, k0, k, moved, swapWith);
+            interchange<BK_THREADS>(F, W, perm, N, k0, k, moved, swapWith);
             if (blockSize == 1)
             {
                 // The pivot column is column imax, its rows k and imax exchanged.
@@ -265,7 +275,409 @@ __global__ __launch_bounds__(BK_THREADS) void bunchKaufmanKernel(const PivotFron
         k += blockSize;
     }
     if (tid == 0)
-        states[q] = PivotState{k, end, passStart, done, twoByTwo, 0, 0, 0};
+        states[q] = PivotState{k, end, passStart, done, twoByTwo, k0, 0, 0};
+}
+
+// The value as an opaque register, in program order: the columns of a panel move down one by one, in place (left to the
+// scheduler, old and new columns overlap and spill).
+__device__ inline double pinned(double v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A workgroup barrier for LDS alone: the stores of L and W in flight need not have landed.
+__device__ inline void ldsBarrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The value a DPP control gives each lane (its own where the control has no source lane).
+template <int CONTROL> __device__ inline double dppValue(double v)
+{
+    const long long bits = __builtin_bit_cast(long long, v);
+    const int lo = int(bits), hi = int(bits >> 32);
+    const unsigned l = unsigned(__builtin_amdgcn_update_dpp(lo, lo, CONTROL, 0xf, 0xf, false));
+    const unsigned h = unsigned(__builtin_amdgcn_update_dpp(hi, hi, CONTROL, 0xf, 0xf, false));
+    return __builtin_bit_cast(double, (static_cast<unsigned long long>(h) << 32) | l);
+}
+
+// The largest value of a wave, in its lane 63 (NaN ignored): shifts by 1, 2, 4 and 8 within rows of 16 lanes, then
+// the rows' last lanes broadcast to the next ones.
+__device__ inline double waveMax(double v)
+{
+    v = fmax(v, dppValue<0x111>(v));
+    v = fmax(v, dppValue<0x112>(v));
+    v = fmax(v, dppValue<0x114>(v));
+    v = fmax(v, dppValue<0x118>(v));
+    v = fmax(v, dppValue<0x142>(v));
+    v = fmax(v, dppValue<0x143>(v));
+    return v;
+}
+
+template <int WAVES> struct PanelShared
+{
+    // By the parity of the column: the waves' largest values, and the column's values in the panel's rows (its diagonal
+    // first).
+    double best[2][WAVES], row[2][PIVOT_PANEL];
+    // Row imax of the panel, updated, and of the step's W; the waves' largest values of column imax, and its diagonal.
+    double line[PIVOT_PANEL], wline[PIVOT_PANEL], rowBest[WAVES], corner;
+    int at;
+};
+
+// A step of one front whose rows from the step's first column k0 on fit R per thread: the columns [k0, k0 + P) lie in
+// registers, thread t holding rows k0 + t + THREADS·r, and are eliminated right-looking; each column done leaves the
+// registers (its L and W stored) as the others move down by one, so the current column is always a[·][0]. A column
+// costs one LDS barrier: the waves' maxima, the diagonal and W's row go through it together. Only the step's first
+// column is interchanged or becomes a 2 × 2 pivot (in memory, where nothing of the step was done yet; the panel is
+// then loaded again): a later column that needs it ends the step and is the next one's first.
+//
+// Bound by the latency of a column (the reduction, a division, the barrier): about 1.4 µs, where columns updated
+// left-looking from L2 (64 to a step, pivotColumnsKernel) took 5 to 30 µs. 16 columns to a step: their product over
+// the trailing candidates reads and writes those once per step, which HBM does beside nothing else (3,600 rows: 16 to
+// 28 µs), so narrower steps pay there; wider ones do not fit the registers (R·P doubles: 128 VGPRs at R·P = 64). The
+// 360 × 200 cylinder's factorisation took 328 ms before and 85 ms with these steps, launched without a wait between.
+template <int THREADS, int R, int P>
+__device__ void eliminatePanel(const PivotFront& fr, PivotState& st, PanelShared<THREADS / 64>& sh)
+{
+    constexpr int WAVES = THREADS / 64;
+    double* F = fr.F;
+    double* W = fr.W;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int64_t N = fr.N;
+    const int n = fr.N, k0 = st.k;
+    int k = k0, end = st.end;
+    int forced = 0; // the first pivot is settled: 1 × 1 or 2 × 2
+    double a[R][P];
+    while (k < end)
+    {
+        const int pc = min(P, end - k0);
+#pragma unroll
+        for (int j = 0; j < P; ++j)
+        {
+            const double* column = F + (k0 + min(j, pc - 1)) * N;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                a[r][j] = column[unsigned(min(k0 + tid + THREADS * r, n - 1))];
+        }
+        if (forced == 2)
+        {
+            // LdltArithmetic's invertTwoByTwo: d11 = c/b, d22 = a/b, t = 1/(d11·d22 − 1), s = t/b.
+            if (tid < pc)
+            {
+                sh.row[0][tid] = a[0][0]; // row k0 + tid
+                sh.row[1][tid] = a[0][1];
+            }
+            __syncthreads();
+            const double d0 = sh.row[0][0], e = sh.row[0][1], d1 = sh.row[1][1];
+            const double d11 = d1 / e, d22 = d0 / e;
+            const double t = 1.0 / (d11 * d22 - 1.0);
+            const double s = t / e;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+            {
+                const int i = k0 + tid + THREADS * r;
+                const double r0 = a[r][0], r1 = a[r][1];
+                const double l0 = s * (d11 * r0 - r1), l1 = s * (d22 * r1 - r0);
+                if (i > k0 + 1 && i < n)
+                {
+                    F[i + k0 * N] = l0;
+                    F[i + (k0 + 1) * N] = l1;
+                    W[i + k0 * N] = r0;
+                    W[i + (k0 + 1) * N] = r1;
+                }
+#pragma unroll
+                for (int j = 2; j < P; ++j)
+                    a[r][j - 2] = pinned(a[r][j] - l0 * sh.row[0][j] - l1 * sh.row[1][j]);
+            }
+            if (tid == 0)
+            {
+                F[k0 + k0 * N] = d0;
+                F[(k0 + 1) + k0 * N] = 0.0;
+                F[(k0 + 1) + (k0 + 1) * N] = d1;
+                fr.diag[k0] = d0;
+                fr.diag[k0 + 1] = d1;
+                fr.sub[k0] = e;
+                fr.sub[k0 + 1] = 0.0;
+            }
+            ++st.twoByTwo;
+            forced = 0;
+            k += 2;
+            __syncthreads(); // the rows are read
+        }
+        bool again = false; // the first column was interchanged, delayed or paired: load and go on
+        while (k < k0 + pc)
+        {
+            const int parity = (k - k0) & 1, left = k0 + pc - k; // the columns still in the panel
+            double m = 0.0;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+            {
+                const int i = k0 + tid + THREADS * r;
+                if (i > k && i < n)
+                    m = fmax(m, fabs(a[r][0]));
+            }
+            const int row = k0 + tid - k;
+            if (row >= 0 && row < left) // the panel's rows: THREADS >= P
+                sh.row[parity][row] = a[0][0];
+            m = waveMax(m);
+            if (lane == 63)
+                sh.best[parity][wave] = m;
+            ldsBarrier();
+            double colmax = sh.best[parity][0];
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w)
+                colmax = fmax(colmax, sh.best[parity][w]);
+            const double d = sh.row[parity][0], absakk = fabs(d);
+            if (forced == 0 && absakk < BK_ALPHA * colmax)
+            {
+                // The first row of the largest value.
+                __syncthreads();
+                if (tid == 0)
+                    sh.at = n;
+                __syncthreads();
+#pragma unroll
+                for (int r = R - 1; r >= 0; --r)
+                {
+                    const int i = k0 + tid + THREADS * r;
+                    if (i > k && i < n && fabs(a[r][0]) == colmax)
+                        atomicMin(&sh.at, i);
+                }
+                __syncthreads();
+                const int imax = sh.at;
+                if (imax >= end)
+                {
+                    if (absakk < BK_DELAY * colmax)
+                    {
+                        // The partner is not a candidate and the diagonal is too small: delay the column.
+                        if (k == k0)
+                        {
+                            --end;
+                            if (k != end)
+                                interchange<THREADS>(F, W, fr.perm, n, k, k, k, end);
+                            again = true;
+                        }
+                        break;
+                    }
+                }
+                else
+                {
+                    // Column imax, updated by the step's columns: its largest value besides its diagonal, and that.
+                    if (tid < k - k0)
+                        sh.wline[tid] = W[imax + (k0 + tid) * N];
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (k0 + tid + THREADS * r == imax)
+                        {
+#pragma unroll
+                            for (int j = 0; j < P; ++j)
+                                sh.line[j] = a[r][j];
+                        }
+                    __syncthreads();
+                    const int at = imax - k;
+                    double rowmax = 0.0;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                    {
+                        const int i = k0 + tid + THREADS * r;
+                        if (i < k || i >= n)
+                            continue;
+                        double v;
+                        if (i < imax && i < k + left)
+                            v = sh.line[i - k];
+                        else if (at < left)
+                        {
+                            v = a[r][0];
+#pragma unroll
+                            for (int j = 1; j < P; ++j)
+                                v = j == at ? a[r][j] : v;
+                        }
+                        else
+                        {
+                            v = i >= imax ? F[i + imax * N] : F[imax + i * N];
+                            constexpr int BATCH = 5; // loads in flight
+                            for (int t0 = k0; t0 < k; t0 += BATCH)
+                            {
+                                double l[BATCH];
+#pragma unroll
+                                for (int t = 0; t < BATCH; ++t)
+                                    l[t] = F[i + min(t0 + t, k - 1) * N];
+#pragma unroll
+                                for (int t = 0; t < BATCH; ++t)
+                                    v = t0 + t < k ? v - pinned(l[t]) * sh.wline[t0 + t - k0] : v;
+                            }
+                        }
+                        if (i == imax)
+                            sh.corner = v;
+                        else
+                            rowmax = fmax(rowmax, fabs(v));
+                    }
+                    rowmax = waveMax(rowmax);
+                    if (lane == 63)
+                        sh.rowBest[wave] = rowmax;
+                    __syncthreads();
+                    rowmax = sh.rowBest[0];
+#pragma unroll
+                    for (int w = 1; w < WAVES; ++w)
+                        rowmax = fmax(rowmax, sh.rowBest[w]);
+                    if (!(absakk >= BK_ALPHA * colmax * (colmax / rowmax)))
+                    {
+                        if (k == k0)
+                        {
+                            forced = fabs(sh.corner) >= BK_ALPHA * rowmax ? 1 : 2;
+                            __syncthreads(); // the tests are read
+                            const int moved = k + forced - 1;
+                            if (imax != moved)
+                                interchange<THREADS>(F, W, fr.perm, n, k, k, moved, imax);
+                            again = true;
+                        }
+                        break;
+                    }
+                }
+            }
+            const bool zero = d == 0.0 && colmax == 0.0; // a zero pivot: nothing to eliminate with it
+            double l[R];
+            double *Fk = F + k * N, *Wk = W + k * N;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+            {
+                const int i = k0 + tid + THREADS * r;
+                l[r] = pinned(zero ? 0.0 : a[r][0] / d);
+                if (i > k && i < n)
+                {
+                    Fk[unsigned(i)] = l[r];
+                    Wk[unsigned(i)] = a[r][0];
+                }
+            }
+#pragma unroll
+            for (int j = 1; j < P; ++j)
+            {
+                const double w = sh.row[parity][j];
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    a[r][j - 1] = pinned(a[r][j] - l[r] * w);
+            }
+            if (tid == 0)
+            {
+                Fk[unsigned(k)] = d;
+                fr.diag[k] = d;
+                fr.sub[k] = 0.0;
+            }
+            forced = 0;
+            ++k;
+        }
+        if (!again)
+            break;
+    }
+    st.from = k0;
+    st.k = k;
+    st.end = end;
+}
+
+// One step of each front of the list, a workgroup per front, for fronts whose remaining rows fit the registers
+// (PIVOT_SMALL_ROWS with 256 threads, PIVOT_LARGE_ROWS with 512).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void pivotPanelKernel(const PivotFront* fronts, PivotState* states,
+                                                            const int32_t* list)
+{
+    __shared__ PanelShared<THREADS / 64> sh;
+    const int q = list[blockIdx.x];
+    const PivotFront fr = fronts[q];
+    PivotState st = states[q];
+    st.from = st.k;
+    if (!st.done && st.k == st.end)
+    {
+        if (st.end == fr.C || st.k == st.passStart)
+            st.done = 1;
+        else
+        {
+            st.passStart = st.k; // another pass over the delayed candidates
+            st.end = fr.C;
+        }
+    }
+    if (!st.done)
+    {
+        const int rows = fr.N - st.k;
+        if (rows <= THREADS)
+            eliminatePanel<THREADS, 1, PIVOT_PANEL>(fr, st, sh);
+        else if (THREADS == 256 || rows <= 2 * THREADS)
+            eliminatePanel<THREADS, 2, PIVOT_PANEL>(fr, st, sh);
+        else if constexpr (THREADS == 512)
+        {
+            if (rows <= 4 * THREADS)
+                eliminatePanel<THREADS, 4, PIVOT_PANEL>(fr, st, sh);
+            else
+                eliminatePanel<THREADS, 8, PIVOT_PANEL / 2>(fr, st, sh);
+        }
+        if (st.k == st.end && (st.end == fr.C || st.k == st.passStart))
+            st.done = 1;
+    }
+    __syncthreads(); // every thread has read the state
+    if (threadIdx.x == 0)
+        states[q] = st;
+}
+
+// The trailing update of the last step: C −= L·Wᵀ over the step's columns [from, k), for the candidate columns and the
+// rows from k on; item {front, row tile, column tile} of 64 × 64 at fixed positions of the front, four waves of
+// 32 × 32 whose MFMA operands come straight from memory (K <= 17: nothing to reuse through LDS). Items whose columns
+// are all eliminated do nothing.
+__global__ __launch_bounds__(256) void pivotTrailingKernel(const PivotFront* fronts, const PivotState* states,
+                                                           const int4* items)
+{
+    const int4 item = items[blockIdx.x];
+    const PivotState st = states[item.x];
+    const PivotFront fr = fronts[item.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row0 = 64 * item.y + 32 * (wave >> 1), col0 = 64 * item.z + 32 * (wave & 1);
+    const int from = st.from, k = st.k, n = fr.N;
+    if (from == k || col0 + 32 <= k || col0 >= fr.C || row0 >= n || row0 + 32 <= max(k, col0))
+        return;
+    const int64_t N = n;
+    const int lr = lane & 15, lq = lane >> 4;
+    double4_t acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int i = min(row0 + 16 * x + lq + 4 * v, n - 1), j = min(col0 + 16 * y + lr, n - 1);
+                acc[x][y][v] = fr.F[i + j * N];
+            }
+    for (int t0 = from; t0 < k; t0 += 4)
+    {
+        const int t = min(t0 + lq, k - 1);
+        double av[2], bv[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+        {
+            av[x] = fr.F[min(row0 + 16 * x + lr, n - 1) + t * N];
+            bv[x] = fr.W[min(col0 + 16 * x + lr, n - 1) + t * N];
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+        {
+            av[x] = t0 + lq < k ? -av[x] : 0.0;
+            bv[x] = t0 + lq < k ? bv[x] : 0.0;
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x], bv[y], acc[x][y], 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int i = row0 + 16 * x + lq + 4 * v, j = col0 + 16 * y + lr;
+                if (i < n && j < fr.C && i >= j && j >= k)
+                    fr.F[i + j * N] = acc[x][y][v];
+            }
 }
 
 // The matrix entries of each front's own columns, at their positions (rows past the own columns move down by the
@@ -394,14 +806,27 @@ int rowGroups(int64_t n)
 
 } // namespace
 
-hipError_t launchBunchKaufman(const PivotFront* fronts, PivotState* states, const int32_t* list, int count, int nb,
-                              hipStream_t stream)
+hipError_t launchPivotStep(int kind, const PivotFront* fronts, PivotState* states, const int32_t* list, int count,
+                           hipStream_t stream)
 {
     if (count == 0)
         return hipSuccess;
-    if (nb < 1 || nb > 2 * PANEL_BLOCK)
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bunchKaufmanKernel, dim3(count), dim3(BK_THREADS), 0, stream, fronts, states, list, nb);
+    if (kind == PIVOT_SMALL)
+        hipLaunchKernelGGL(pivotPanelKernel<256>, dim3(count), dim3(256), 0, stream, fronts, states, list);
+    else if (kind == PIVOT_LARGE)
+        hipLaunchKernelGGL(pivotPanelKernel<512>, dim3(count), dim3(512), 0, stream, fronts, states, list);
+    else
+        hipLaunchKernelGGL(pivotColumnsKernel, dim3(count), dim3(BK_THREADS), 0, stream, fronts, states, list,
+                           PIVOT_PANEL);
+    return hipGetLastError();
+}
+
+hipError_t launchPivotTrailing(const PivotFront* fronts, const PivotState* states, const int4* items, int count,
+                               hipStream_t stream)
+{
+    if (count == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(pivotTrailingKernel, dim3(count), dim3(256), 0, stream, fronts, states, items);
     return hipGetLastError();
 }
 

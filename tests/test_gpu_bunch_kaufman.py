@@ -170,3 +170,92 @@ def test_dense_front_matches_the_oracle_bunch_kaufman(gpu_device, n, seed):
     b = rng.standard_normal((n, 2))
     x = FactorSolve(f).solve(b)
     assert np.max(np.abs(dense @ x - b)) <= 1e-9 * (np.max(np.abs(dense)) * np.max(np.abs(x)) + np.max(np.abs(b)))
+
+
+def dense_problem(dense):
+    """One supernode whose front is the whole matrix: (symbolic factor, matrix)."""
+    n = dense.shape[0]
+    sym = SymbolicFactor(n, [0], [n], [-1], [0, 0], np.zeros(0, np.int32))
+    rows = np.concatenate([np.arange(j, n) for j in range(n)]).astype(np.int32)
+    offsets = np.concatenate([[0], np.cumsum(np.arange(n, 0, -1))]).astype(np.int64)
+    return sym, SymmetricCsc(n, offsets, rows, np.concatenate([dense[j:, j] for j in range(n)]))
+
+
+@pytest.mark.parametrize("n,diagonal", [(1, 1.0), (16, 1e-3), (17, 30.0), (64, 10.0), (512, 50.0), (513, 1e-3),
+                                        (1025, 50.0)])
+def test_panel_edges_match_the_oracle_bunch_kaufman(gpu_device, n, diagonal):
+    # The steps' panels at the edges of their register layouts (16 columns; 256, 512 and 1024 rows), with diagonals
+    # that make almost every pivot 2 × 2 (1e-3) or pass most tests and interchange some columns (10 to 50): the oracle's
+    # pivots exactly. Values: n·eps·(growth of the pivots, up to 1e3 here) is below 1e-9.
+    rng = np.random.default_rng(n)
+    dense = rng.standard_normal((n, n))
+    dense = dense + dense.T
+    dense[np.arange(n), np.arange(n)] *= diagonal
+    sym, m = dense_problem(dense)
+    f = SupernodalFactor.factorise(sym, m, INDEFINITE)
+    a = np.array(np.tril(dense), order="F")
+    perm, sub = np.zeros(n, np.int64), np.zeros(n)
+    assert _oracle.oracle().orc_bunch_kaufman(_oracle.P(a), n, n, n, _oracle.P(perm), _oracle.P(sub)) == n
+    values, rows = f.panel(0)
+    assert rows.tolist() == perm.tolist()
+    assert np.array_equal(f.subdiagonal(0) != 0, sub != 0)
+    assert np.max(np.abs(np.tril(values, -1) - np.tril(a, -1))) <= 1e-9 * max(1.0, np.max(np.abs(np.tril(a, -1))))
+    assert np.max(np.abs(np.diag(values) - np.diag(a))) <= 1e-9 * np.max(np.abs(np.diag(a)))
+
+
+@pytest.mark.parametrize("columns,rows", [(20, 1030), (3, 2046), (33, 4090), (5, 4100)])
+def test_tall_fronts_keep_their_inertia(gpu_device, columns, rows):
+    # A supernode of few columns over many rows and its parent, at the row counts where the panel takes another layout
+    # (1024, 2048, 4096 rows) or the columns go through memory (more): a diagonal that dominates with random signs is
+    # its own pivot order (no interchange), and its signs are the inertia.
+    n = columns + rows
+    sym = SymbolicFactor(n, [0, columns], [columns, rows], [1, -1], [0, rows, rows],
+                         np.arange(columns, n, dtype=np.int32))
+    rng = np.random.default_rng(n)
+    dense = np.tril(rng.uniform(-1.0, 1.0, (n, n)), -1)
+    signs = np.where(rng.random(n) < 0.3, -1.0, 1.0)
+    dense[np.arange(n), np.arange(n)] = signs * n
+    _, m = dense_problem(dense)
+    f = SupernodalFactor.factorise(sym, m, INDEFINITE)
+    assert [f.inertia.positive, f.inertia.negative, f.inertia.zero] == [int(np.sum(signs > 0)), int(np.sum(signs < 0)),
+                                                                      0]
+    assert f.panel(0)[1].tolist() == list(range(n)) and f.two_by_two_pivot_count == 0
+    b = rng.standard_normal((n, 2))
+    x = FactorSolve(f).solve(b)
+    full = dense + np.tril(dense, -1).T
+    assert np.max(np.abs(full @ x - b)) <= 1e-13 * (np.max(np.sum(np.abs(full), 1)) * np.max(np.abs(x)) +
+                                                     np.max(np.abs(b)))
+
+
+@pytest.mark.parametrize("sizes,seed", [((5, 7, 6), 1), ((70, 90, 40), 3), ((300, 420, 200), 5)])
+def test_delayed_columns_keep_the_inertia(gpu_device, sizes, seed):
+    # Two cliques whose own couplings are tiny against those to a separator: their columns are delayed into its front
+    # (passes that eliminate nothing, fronts that grow). The inertia is that of the dense eigenvalues, which lie far
+    # from zero.
+    groups = np.split(np.arange(sum(sizes)), np.cumsum(sizes)[:-1])
+    graph = clique_graph([g.tolist() for g in groups], [(0, 2), (1, 2)])
+    n = sum(sizes)
+    sym = SymbolicFactor.analyse(graph[0], graph[1], graph[2], np.arange(n, dtype=np.int32))
+    assert sym.node_order.tolist() == list(range(n))
+    rng = np.random.default_rng(seed)
+    group_of = np.repeat([0, 1, 2], sizes)
+    dense = np.tril(rng.standard_normal((n, n)))
+    weak = (group_of[:, None] == group_of[None, :]) & (group_of[:, None] < 2)
+    dense = np.where(weak, 1e-4 * dense, dense)
+    dense[np.arange(n), np.arange(n)] *= np.where(group_of < 2, 0.1, 1.0)
+    dense[(group_of[:, None] + group_of[None, :]) == 1] = 0.0  # the two cliques do not touch
+    offsets, rows, values = [0], [], []
+    for j in range(n):
+        below = [j] + [int(i) for i in graph[1][graph[0][j]:graph[0][j + 1]] if i > j]
+        rows += below
+        values += dense[below, j].tolist()
+        offsets.append(len(rows))
+    m = SymmetricCsc(n, np.array(offsets), np.array(rows, np.int32), np.array(values))
+    full = m.to_dense()
+    f = SupernodalFactor.factorise(sym, m, INDEFINITE)
+    eigenvalues = np.linalg.eigvalsh(full)
+    assert f.delayed_pivot_count > 0
+    assert (f.inertia.negative, f.inertia.positive) == (int(np.sum(eigenvalues < 0)), int(np.sum(eigenvalues > 0)))
+    b = rng.standard_normal((n, 2))
+    x = FactorSolve(f).solve(b)
+    assert backward_error(m, x, b) <= 1e-12
