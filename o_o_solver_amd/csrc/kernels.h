@@ -70,11 +70,21 @@ struct AssemblyItem
 // An update-matrix tile of extendTilesKernel (64 × 64 or 128 × 128) also adds its children's contributions: its
 // 64 × 64 quarters q take the assembly items [itemStarts[items + q], itemStarts[items + q + 1]); rowBase and colBase are
 // the front positions of its element (0, 0).
+// Mode 2 (a mode-0 tile on the diagonal whose update finishes the next panel step's block, factorised there): ldb is
+// the offset of the block's inverse, items the equation of its first column, rowBase that column, colBase its width.
 struct UpdateTile
 {
     int64_t cOff, aOff, bOff, dOff, ld, ldb, ldc;
     int32_t m, n, k, target, lower, mode;
     int32_t items, supernode, rowBase, colBase;
+};
+
+// The first diagonal block of a front's panel (element offsets): its order n, its width kb, the equation of its first
+// column.
+struct DiagonalBlock
+{
+    int64_t panel, linv;
+    int32_t n, kb, first, supernode;
 };
 
 // A pivoted front of the indefinite factorisation (device pointers): F, N × N column-major, positions [own columns c,
@@ -189,8 +199,8 @@ template <typename T>
 hipError_t launchAssembly(const DevicePlan& p, const DeviceMatrix& a, T* panels, T* updates,
                           const AssemblyBlock* blocks, const AssemblyItem* items, int count, hipStream_t stream);
 template <typename T>
-hipError_t launchDiagonalBlocks(const DevicePlan& p, T* panels, T* linv, const int32_t* fronts, int frontCount, int k0,
-                                double* diagOut, int32_t* zeroAt, hipStream_t stream);
+hipError_t launchDiagonalBlocks(T* panels, T* linv, const DiagonalBlock* blocks, int count, double* diagOut,
+                                int32_t* zeroAt, hipStream_t stream);
 // A step of the whole inverses X = L_FF⁻¹ of the wide supernodes' triangles (items (s, I << 16 | J)): step K >= 0
 // updates T_IJ = −Σ_{K'<=K} L_IK'·X_K'J for I > K >= J; step −1 sets X_IJ = L_II⁻¹·T_IJ (I > J) and X_II = L_II⁻¹.
 template <typename T>

@@ -385,20 +385,6 @@ __global__ __launch_bounds__(256) void assembleKernel(DevicePlan p, DeviceMatrix
     });
 }
 
-// The value of lane `lane` (uniform across the wave) on every lane: v_readlane into a scalar register, a few cycles,
-// where a general shuffle (ds_bpermute) waits on LDS latency.
-__device__ inline float broadcastLane(float v, int lane)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-__device__ inline double broadcastLane(double v, int lane)
-{
-    const long long bits = __builtin_bit_cast(long long, v);
-    const unsigned lo = unsigned(__builtin_amdgcn_readlane(int(bits), lane));
-    const unsigned hi = unsigned(__builtin_amdgcn_readlane(int(bits >> 32), lane));
-    return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
-}
-
 // MFMA tiles, 64 × 64 per workgroup, four waves of 32 × 32 in 16 × 16 × 4 blocks:
 //   mode 0  C −= A·diag(d)·Bᵀ  the trailing update of a panel step, and the update matrix of a front;
 //   mode 1  C  = A·Bᵀ·diag(d)⁻¹ with B = L11⁻¹ of the diagonal block: the panel solve (rows below a factorised
@@ -408,41 +394,46 @@ __device__ inline double broadcastLane(double v, int lane)
 
 // The diagonal block [k0, k0 + kb) of a front's panel factorised in place (kb <= PANEL_BLOCK), with the inverse of
 // its unit lower factor; one workgroup of four waves per front, the block in LDS (rows and columns from kb on hold
-// the identity, which the elimination leaves unchanged):
-//   elimination by sub-panels of 16 columns: wave 0 eliminates the sub-panel's columns one after the other, a row per
-//     lane, the pivot d_k and W(j, k) = L(j, k)·d_k broadcast from their lanes by v_readlane (the reference's chain,
-//     DenseBlockKernels.cpp:376-390, inside the sub-panel); then the waves subtract L·W of the sub-panel from the
-//     trailing lower 16 × 16 tiles with MFMA;
-//   inverse X = L⁻¹: the four diagonal tiles by forward substitution (wave w: X_ww, lane j its column j), then the
-//     tiles below, by distance d = I − J = 1, 2, 3: X_IJ = −X_II·(Σ_{K=J}^{I−1} L_IK·X_KJ), two MFMA products, the
-//     first one's accumulator used directly as the second one's operand (its k-steps follow the accumulator rows).
+// the identity, which the elimination leaves unchanged), by sub-panels of 16 columns P:
+//   elimination of the sub-panel's diagonal tile P by wave 0, which holds it (both triangles) a column per lane of each
+//     group of 16, with the identity beside it: row v takes −a(v, k)·(row k / d_k), a(v, k) and the pivot broadcast
+//     within the group by DPP (the reference's chain, DenseBlockKernels.cpp:376-390, the division on the other factor
+//     of each product); the identity's rows take −L(v, k)·(row k) and become X_PP = L_PP⁻¹;
+//   the tiles below, W_IP = A_IP·X_PPᵀ and L_IP = W_IP·D⁻¹, then the trailing lower tiles A_IJ −= L_IP·W_JPᵀ, MFMA
+//     products spread over the waves;
+//   inverse X = L⁻¹: wave J + 1 its column of tiles J, while wave 0 eliminates: X_PJ = −X_PP·T with
+//     T = Σ_{K=J}^{P−1} L_PK·X_KJ summed ahead; T's accumulator is the second product's operand as it is (its k-steps
+//     follow the accumulator rows).
+// Bound by the chain of the 64 pivots, one wave's (a broadcast, a division and a product each: 210 cycles with the
+// products beside them), and the stores. A block of 64 takes 16 µs standalone and 20.5 µs in an update launch (FP64);
+// with the columns eliminated a row per lane over the 64 rows (15 broadcasts of W by v_readlane a column) and the
+// inverse after the elimination 26 and 32 µs.
 // LDS: S[j·LD + i] holds L(i, j) for i > j, D(j) for i = j, and X(j, i) for i < j (the inverse, transposed, in the
 // upper triangle, which the elimination leaves free).
 // Factors the block held in S (LD = PANEL_BLOCK + 1: S[j·LD + i] = F(k0 + i, k0 + j) for i >= j, the identity
-// outside the kb × kb block) and writes it back: L and D into the panel, L11⁻¹ into the inverses, D into diagOut; a
-// zero or non-finite pivot is recorded in zeroAt. One workgroup of four waves.
+// outside the kb × kb block) and writes it back: L and D into the panel (`block`, leading dimension n), L11⁻¹ to `out`,
+// D to `diag`; a zero or non-finite pivot is recorded in *zeroAt (its column, the block's first being k0). One workgroup
+// of four waves. The places come with the tile or the block's descriptor: read from the plan's arrays here, each is a
+// wait on memory after the elimination.
 template <typename T>
-__device__ void factorBlockInLds(T* S, const DevicePlan& p, int s, int k0, int kb, T* panels, T* linv,
-                                 double* diagOut, int32_t* zeroAt);
+__device__ __forceinline__ void factorBlockInLds(T* S, int kb, int k0, int n, T* block, T* out, double* diag, int32_t* zeroAt);
 
 template <typename T>
-__global__ __launch_bounds__(256, 2) void diagonalBlockKernel(DevicePlan p, T* panels, T* linv, const int32_t* list,
-                                                           int k0, double* diagOut, int32_t* zeroAt)
+__global__ __launch_bounds__(256, 2) void diagonalBlockKernel(T* panels, T* linv, const DiagonalBlock* blocks,
+                                                              double* diagOut, int32_t* zeroAt)
 {
     constexpr int B = PANEL_BLOCK, LD = PANEL_BLOCK + 1;
     __shared__ T S[B * LD];
-    const int s = list[blockIdx.x];
-    const int c = p.ncol[s], n = c + p.nrow[s];
-    const int kb = min(B, c - k0);
-    T* panel = panels + p.panelOff[s];
+    const DiagonalBlock d = blocks[blockIdx.x];
+    const int n = d.n, kb = d.kb;
+    T* const block = panels + d.panel;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int64_t base = k0 + int64_t(k0) * n;
 
     // Every load is issued (from the block's first element where the position is outside the lower triangle) and
     // the value selected afterwards: no branch waits on an earlier load.
     // Thread (wave, lane) moves rows i = lane of the columns j = wave + 4q.
     {
-        const T* src = panel + base + int64_t(wave) * n;
+        const T* src = block + int64_t(wave) * n;
         T v[B / 4];
 #pragma unroll
         for (int q = 0; q < B / 4; ++q)
@@ -450,7 +441,7 @@ __global__ __launch_bounds__(256, 2) void diagonalBlockKernel(DevicePlan p, T* p
             // Columns from kb on lie outside the panel (past the end of the panel array for the last supernode):
             // their loads read the block's first element instead.
             const int j = wave + 4 * q;
-            const T* column = j < kb ? src : panel + base;
+            const T* column = j < kb ? src : block;
             v[q] = column[(lane < kb && j < kb && lane >= j) ? lane : 0];
             src += 4 * int64_t(n);
         }
@@ -463,161 +454,424 @@ __global__ __launch_bounds__(256, 2) void diagonalBlockKernel(DevicePlan p, T* p
         }
     }
     __syncthreads();
-    factorBlockInLds(S, p, s, k0, kb, panels, linv, diagOut, zeroAt);
+    factorBlockInLds(S, kb, 0, n, block, linv + d.linv, diagOut + d.first, zeroAt + d.supernode);
+}
+
+// N registers plus m times the lane K of each group of 16 lanes of themselves (addOwnBroadcasts), or the register V + e
+// plus y times the lane V + e of each group of m (addBroadcasts). Each block starts with the two wait states that a DPP
+// source needs after the instruction that wrote it.
+template <int K, int N> __device__ inline void addOwnBroadcasts(double* acc, double m)
+{
+    if constexpr (N == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %0, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %1, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %2, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %3, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %4, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %5, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %6, %6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %7, %7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]),
+              "+&v"(acc[6]), "+&v"(acc[7])
+            : "v"(m), "n"(K));
+    else if constexpr (N == 4)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])
+            : "v"(m), "n"(K));
+    else if constexpr (N == 2)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1])
+            : "v"(m), "n"(K));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0])
+            : "v"(m), "n"(K));
+}
+template <int V, int N> __device__ inline void addBroadcasts(double* acc, double m, double y)
+{
+    if constexpr (N == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %4, %8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %5, %8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %6, %8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %7, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]),
+              "+&v"(acc[6]), "+&v"(acc[7])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1), "n"(V + 2), "n"(V + 3), "n"(V + 4), "n"(V + 5),
+              "n"(V + 6), "n"(V + 7));
+    else if constexpr (N == 4)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1), "n"(V + 2), "n"(V + 3));
+    else if constexpr (N == 2)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0])
+            : "v"(m), "v"(y), "n"(V));
+}
+template <int K, int N> __device__ inline void addOwnBroadcasts(float* acc, float m)
+{
+    if constexpr (N == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %0, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %1, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %2, %2, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %3, %3, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %4, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %5, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %6, %6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %7, %7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]),
+              "+&v"(acc[6]), "+&v"(acc[7])
+            : "v"(m), "n"(K));
+    else if constexpr (N == 4)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])
+            : "v"(m), "n"(K));
+    else if constexpr (N == 2)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1])
+            : "v"(m), "n"(K));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0])
+            : "v"(m), "n"(K));
+}
+template <int V, int N> __device__ inline void addBroadcasts(float* acc, float m, float y)
+{
+    if constexpr (N == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %2, %8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %3, %8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %4, %8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %5, %8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %6, %8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %7, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]),
+              "+&v"(acc[6]), "+&v"(acc[7])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1), "n"(V + 2), "n"(V + 3), "n"(V + 4), "n"(V + 5),
+              "n"(V + 6), "n"(V + 7));
+    else if constexpr (N == 4)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1), "n"(V + 2), "n"(V + 3));
+    else if constexpr (N == 2)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0]), "+&v"(acc[1])
+            : "v"(m), "v"(y), "n"(V), "n"(V + 1));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+&v"(acc[0])
+            : "v"(m), "v"(y), "n"(V));
+}
+
+// The lane K of each group of 16 lanes of v, on every lane of the group.
+template <int K> __device__ inline double groupBroadcast(double v)
+{
+    double out;
+    asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(out) : "v"(v), "n"(K));
+    return out;
+}
+template <int K> __device__ inline float groupBroadcast(float v)
+{
+    float out;
+    asm("s_nop 1\n\tv_mov_b32_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(out) : "v"(v), "n"(K));
+    return out;
+}
+
+// The rows [V, 16) of a tile in registers: a's plus m times their lane K, x's plus y times the lane of their number of m.
+template <typename T, int K, int V> __device__ inline void addOwnRows(T (&a)[16], T m)
+{
+    if constexpr (V < 16)
+    {
+        constexpr int N = V % 8 == 0 ? 8 : (V % 4 == 0 ? 4 : (V % 2 == 0 ? 2 : 1));
+        addOwnBroadcasts<K, N>(a + V, m);
+        addOwnRows<T, K, V + N>(a, m);
+    }
+}
+template <typename T, int V> __device__ inline void addRows(T (&x)[16], T m, T y)
+{
+    if constexpr (V < 16)
+    {
+        constexpr int N = V % 8 == 0 ? 8 : (V % 4 == 0 ? 4 : (V % 2 == 0 ? 2 : 1));
+        addBroadcasts<V, N>(x + V, m, y);
+        addRows<T, V + N>(x, m, y);
+    }
+}
+
+// The columns K .. 15 of a 16 × 16 tile eliminated in one wave's registers: lane j of each group of 16 holds column j,
+// row v in a[v] (W = L·D below the diagonal, the pivots on it; above it, working values), and column j of the identity,
+// which becomes L⁻¹, in x. L(v, K) is −m of lane v. No branch: the identity's columns beyond a block leave the others
+// as they are.
+template <typename T, int K> __device__ inline void eliminateTile(T (&a)[16], T (&x)[16], int j)
+{
+    if constexpr (K < 15)
+    {
+        const T pivot = groupBroadcast<K>(a[K]);
+        const T m = (j > K ? -a[K] : T(0)) / pivot;
+        addOwnRows<T, K, K + 1>(a, m);
+        addRows<T, K + 1>(x, m, x[K]);
+        eliminateTile<T, K + 1>(a, x, j);
+    }
+}
+
+// The tile (I, J) less L·W of the sub-panel P (16 × 16 tiles of the block in S: LD and S as in factorBlockInLds). The
+// rows beyond the block hold the identity, which the update (with L zero there) leaves as it is.
+template <typename T> __device__ inline void updateTile(T* S, int P, int I, int J, int lane)
+{
+    constexpr int LD = PANEL_BLOCK + 1, SP = 16;
+    const int m = lane & 15, g = lane >> 4, col = SP * J + m;
+    T av[4], bv[4], dv[4];
+    typename Mfma<T>::Acc acc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+    {
+        const int pc = SP * P + 4 * e + g;
+        acc[e] = S[col * LD + SP * I + Mfma<T>::row(lane, e)];
+        av[e] = S[pc * LD + SP * I + m];
+        bv[e] = S[pc * LD + col];
+        dv[e] = S[pc * LD + pc];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        acc = Mfma<T>::step(-av[e], bv[e] * dv[e], acc);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        S[col * LD + SP * I + Mfma<T>::row(lane, v)] = acc[v];
+}
+
+// Σ_{K=J}^{P−1} L_PK·X_KJ (16 × 16 tiles of the block in S: LD and S as in factorBlockInLds).
+template <typename T> __device__ inline typename Mfma<T>::Acc inverseTerms(const T* S, int P, int J, int lane)
+{
+    constexpr int LD = PANEL_BLOCK + 1, SP = 16;
+    const int m = lane & 15, g = lane >> 4;
+    typename Mfma<T>::Acc t = {0, 0, 0, 0};
+    for (int K = J; K < P; ++K)
+    {
+        T av[4], bv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            const int rk = SP * K + 4 * q + g, cj = SP * J + m;
+            av[q] = S[rk * LD + SP * P + m]; // L(16P + m, rk)
+            bv[q] = S[rk * LD + cj];         // X(rk, cj) below the diagonal
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            const int rk = SP * K + 4 * q + g, cj = SP * J + m;
+            const T b = pinned(bv[q]);
+            t = Mfma<T>::step(pinned(av[q]), rk > cj ? b : T(rk == cj ? 1 : 0), t);
+        }
+    }
+    return t;
+}
+
+// X_PJ = −X_PP·t into S.
+template <typename T>
+__device__ inline void finishInverseTile(T* S, int P, int J, typename Mfma<T>::Acc t, int lane)
+{
+    constexpr int LD = PANEL_BLOCK + 1, SP = 16;
+    const int m = lane & 15;
+    T xv[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        xv[v] = S[(SP * P + m) * LD + SP * P + Mfma<T>::row(lane, v)]; // X_PP(m, ·) below the diagonal
+    typename Mfma<T>::Acc u = {0, 0, 0, 0};
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+    {
+        const int kr = Mfma<T>::row(lane, v);
+        const T x = pinned(xv[v]);
+        u = Mfma<T>::step(m > kr ? x : T(m == kr ? 1 : 0), t[v], u);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        S[(SP * P + Mfma<T>::row(lane, v)) * LD + SP * J + m] = -u[v];
+}
+
+// The strictly lower part of the diagonal tile P divided by its pivots, by one wave: lane (g, i) row i of the columns
+// g + 4q.
+template <typename T> __device__ inline void scaleDiagonalTile(T* S, int P, int lane)
+{
+    constexpr int LD = PANEL_BLOCK + 1, SP = 16;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+    {
+        const int col = SP * P + (lane >> 4) + 4 * q, row = SP * P + (lane & 15);
+        if (row > col)
+            S[col * LD + row] = S[col * LD + row] / S[col * LD + col];
+    }
 }
 
 template <typename T>
-__device__ void factorBlockInLds(T* S, const DevicePlan& p, int s, int k0, int kb, T* panels, T* linv,
-                                 double* diagOut, int32_t* zeroAt)
+__device__ __forceinline__ void factorBlockInLds(T* S, int kb, int k0, int n, T* block, T* out, double* diag, int32_t* zeroAt)
 {
     constexpr int B = PANEL_BLOCK, LD = PANEL_BLOCK + 1, SP = 16;
     static_assert(B == 64, "four sub-panels of 16 columns");
     typedef typename Mfma<T>::Acc Acc;
-    const int c = p.ncol[s], n = c + p.nrow[s];
-    T* panel = panels + p.panelOff[s];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int64_t base = k0 + int64_t(k0) * n;
 
-    for (int c0 = 0; c0 < kb; c0 += SP)
+    const int last = (kb - 1) / SP, J = wave - 1;
+    const int m = lane & 15, g = lane >> 4;
+    Acc t = {0, 0, 0, 0}; // wave J + 1: the terms of the next tile of its column of the inverse
+    for (int P = 0; P <= last; ++P)
     {
+        const int c0 = SP * P;
         if (wave == 0)
         {
-            T a[SP]; // row `lane` of the sub-panel
+            T a[SP], x[SP];
+            T* const column = S + (c0 + m) * LD + c0;
+            T* const row = S + c0 * LD + c0 + m;
 #pragma unroll
-            for (int t = 0; t < SP; ++t)
-                a[t] = S[(c0 + t) * LD + lane];
-#pragma unroll
-            for (int k = 0; k < SP; ++k)
+            for (int v = 0; v < SP; ++v)
             {
-                const int K = c0 + k;
-                if (K >= kb)
-                    break; // the identity beyond the block: nothing to eliminate
-                const T pivot = broadcastLane(a[k], K);
-                if (lane == 0 && isBadPivot(pivot))
-                    atomicMin(&zeroAt[s], k0 + K);
-                const T l = a[k] / pivot; // L(lane, K) on the lanes below K
-                const T w = l * pivot;
-#pragma unroll
-                for (int t = k + 1; t < SP; ++t)
-                    a[t] -= l * broadcastLane(w, c0 + t);
-                if (lane > K)
-                    a[k] = l;
+                a[v] = *(v < m ? row + v * LD : column + v);
+                x[v] = T(v == m ? 1 : 0);
             }
-#pragma unroll
-            for (int t = 0; t < SP; ++t)
-                if (lane >= c0 + t)
-                    S[(c0 + t) * LD + lane] = a[t];
-        }
-        __syncthreads();
-        // Trailing tiles (I, J), c0/16 < J <= I < 4, in the order J, then I; those whose rows lie beyond the block
-        // hold the identity, which the update (with L zero there) leaves as it is.
-        const int P = c0 / SP;
-        const int tiles = (3 - P) * (4 - P) / 2;
-        for (int q = wave; q < tiles; q += 4)
-        {
-            int J = P + 1, I = q;
-            while (I >= 4 - J)
-            {
-                I -= 4 - J;
-                ++J;
-            }
-            I += J;
-            if (SP * I >= kb)
-                continue;
-            const int col = SP * J + (lane & 15);
-            Acc acc;
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                acc[v] = S[col * LD + SP * I + Mfma<T>::row(lane, v)];
-#pragma unroll
-            for (int kk = 0; kk < SP; kk += 4)
-            {
-                const int pc = c0 + kk + (lane >> 4);
-                const T av = -S[pc * LD + SP * I + (lane & 15)];
-                const T bv = S[pc * LD + col] * S[pc * LD + pc];
-                acc = Mfma<T>::step(av, bv, acc);
-            }
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                S[col * LD + SP * I + Mfma<T>::row(lane, v)] = acc[v];
-        }
-        __syncthreads();
-    }
-
-    // Diagonal tiles of the inverse: lane j (lanes from 16 on repeat lane j mod 16 and store nothing); a tile beyond
-    // the block is the identity's, whose inverse's zeros the upper triangle already holds.
-    if (SP * wave < kb)
-    {
-        const int J0 = SP * wave, j = lane & 15;
-        T x[SP];
-#pragma unroll
-        for (int i = 0; i < SP; ++i)
-            x[i] = T(i == j ? 1 : 0);
-#pragma unroll
-        for (int k = 0; k < SP; ++k)
-        {
-#pragma unroll
-            for (int i = k + 1; i < SP; ++i)
-                x[i] -= S[(J0 + k) * LD + J0 + i] * x[k];
-            asm volatile("" ::: "memory"); // one column's reads in flight at a time (registers)
-        }
-        if (lane < SP)
-        {
-#pragma unroll
-            for (int i = 1; i < SP; ++i)
-                if (i > j)
-                    S[(J0 + i) * LD + J0 + j] = x[i];
-        }
-    }
-    __syncthreads();
-    for (int d = 1; d < 4; ++d)
-    {
-        // Tiles whose rows lie beyond the block: L is zero there, and so is X.
-        if (wave < 4 - d && SP * (wave + d) < kb)
-        {
-            const int J = wave, I = wave + d;
-            const int m = lane & 15;
-            Acc t = {0, 0, 0, 0};
-            for (int K = J; K < I; ++K)
+            eliminateTile<T, 0>(a, x, m);
+            // W and D below, X_PP above the diagonal (by one group); a store with no place goes to the column's padding.
+            T* const padding = S + (c0 + m) * LD + B;
+            if (lane < SP)
             {
 #pragma unroll
-                for (int kk = 0; kk < SP; kk += 4)
+                for (int v = 0; v < SP; ++v)
                 {
-                    const int rk = SP * K + kk + (lane >> 4), cj = SP * J + m;
-                    const T av = S[rk * LD + SP * I + m];                                 // L(16I + m, rk)
-                    const T bv = rk > cj ? S[rk * LD + cj] : T(rk == cj ? 1 : 0);           // X(rk, cj)
-                    t = Mfma<T>::step(av, bv, t);
+                    *(v < m ? padding : column + v) = a[v];
+                    if (v > 0)
+                        *(v > m ? row + v * LD : padding) = x[v];
                 }
             }
-            Acc u = {0, 0, 0, 0};
+        }
+        else if (P > 0)
+        {
+            // The last sub-panel's update of the tiles right of column P, at most three of them.
+            const int It = wave == 1 ? P + 1 : P + 2, Jt = wave == 3 ? P + 2 : P + 1;
+            if (SP * It < kb)
+                updateTile(S, P - 1, It, Jt, lane);
+            if (J < P - 1)
+                finishInverseTile(S, P - 1, J, t, lane);
+            if (J < P)
+                t = inverseTerms(S, P, J, lane);
+            if (wave == 3)
+                scaleDiagonalTile(S, P - 1, lane);
+        }
+        __syncthreads();
+        // The tiles below (those beyond the block hold the identity's zeros).
+        if (SP * (P + 1 + wave) < kb)
+        {
+            const int I = P + 1 + wave;
+            T av[4], xv[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
+            for (int q = 0; q < 4; ++q)
             {
-                const int kr = Mfma<T>::row(lane, v);
-                const T xv = m > kr ? S[(SP * I + m) * LD + SP * I + kr] : T(m == kr ? 1 : 0); // X_II(m, kr)
-                u = Mfma<T>::step(xv, t[v], u);
+                av[q] = S[(c0 + 4 * q + g) * LD + SP * I + m];
+                xv[q] = S[(c0 + m) * LD + c0 + 4 * q + g]; // X_PP(m, 4q + g) below the diagonal
+            }
+            const T d = S[(c0 + m) * LD + c0 + m];
+            Acc w = {0, 0, 0, 0};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const T x = pinned(xv[q]);
+                w = Mfma<T>::step(pinned(av[q]), m > 4 * q + g ? x : T(m == 4 * q + g ? 1 : 0), w);
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v)
-                S[(SP * I + Mfma<T>::row(lane, v)) * LD + SP * J + m] = -u[v];
+                S[(c0 + m) * LD + SP * I + Mfma<T>::row(lane, v)] = w[v] / d;
         }
         __syncthreads();
+        // The next sub-panel's tiles (I, P + 1); the trailing tiles after them while it is eliminated.
+        if (SP * (P + 1 + wave) < kb)
+            updateTile(S, P, P + 1 + wave, P + 1, lane);
+        if (P < last)
+            __syncthreads();
     }
+    if (wave == 0)
+        scaleDiagonalTile(S, last, lane);
+    else if (J < last)
+        finishInverseTile(S, last, J, t, lane);
+    __syncthreads();
 
-    T* out = linv + p.linvOff[s] + int64_t(k0) * B;
-    T* dst = panel + base + int64_t(wave) * n;
-    for (int j = wave; j < kb; j += 4)
+    // Wave w writes the columns w + 4q of the panel and of the inverse. A full block's are written whole, without a
+    // branch (the panel's part above the diagonal is never read): masked stores cost a branch each, 260 cycles a column
+    // against 90.
+    if (kb == B)
     {
-        if (lane < kb)
+        constexpr int BATCH = 8;
+#pragma unroll
+        for (int q0 = 0; q0 < B / 4; q0 += BATCH)
         {
-            if (lane >= j)
-                dst[lane] = S[j * LD + lane];
-            out[lane + j * kb] = lane == j ? T(1) : (lane > j ? S[lane * LD + j] : T(0));
+            T l[BATCH], x[BATCH];
+#pragma unroll
+            for (int q = 0; q < BATCH; ++q)
+            {
+                const int j = wave + 4 * (q0 + q);
+                l[q] = S[j * LD + lane];
+                x[q] = S[lane * LD + j];
+            }
+#pragma unroll
+            for (int q = 0; q < BATCH; ++q)
+            {
+                const int j = wave + 4 * (q0 + q);
+                (block + j * int64_t(n))[unsigned(lane)] = pinned(l[q]);
+                (out + j * B)[unsigned(lane)] = lane > j ? pinned(x[q]) : T(lane == j ? 1 : 0);
+            }
         }
-        dst += 4 * int64_t(n);
     }
+    else
+        for (int j = wave; j < kb; j += 4)
+            if (lane < kb)
+            {
+                if (lane >= j)
+                    block[lane + j * int64_t(n)] = S[j * LD + lane];
+                out[lane + j * kb] = lane == j ? T(1) : (lane > j ? S[lane * LD + j] : T(0));
+            }
     if (tid < kb)
-        diagOut[p.first[s] + k0 + tid] = double(S[tid * LD + tid]);
+    {
+        const T d = S[tid * LD + tid];
+        if (isBadPivot(d))
+            atomicMin(zeroAt, k0 + tid);
+        diag[tid] = double(d);
+    }
 }
 
 constexpr int TILE = 64;
@@ -659,7 +913,7 @@ __global__ __launch_bounds__(256, FUSE ? 2 : 1) void updateTilesKernel(DevicePla
     const T* Bm = (solve || PLAIN ? linv : panels) + t.bOff;
     const T* dv = panels + t.dOff;
     const int64_t ld = t.ld, ldb = solve || PLAIN ? t.ldb : t.ld;
-    T* C = (PLAIN || t.target == 0 ? panels : updates) + t.cOff;
+    T* const C = (PLAIN || t.target == 0 ? panels : updates) + t.cOff;
 
     typename Mfma<T>::Acc acc[2][2];
 #pragma unroll
@@ -685,33 +939,35 @@ __global__ __launch_bounds__(256, FUSE ? 2 : 1) void updateTilesKernel(DevicePla
         for (int b = 0; b < 2; ++b)
             pivots[b] = dv[min(wn + b * 16 + (lane & 15), t.n - 1) * (ld + 1)];
     }
-    T ra[PER], rb[PER], rd[PER];
-    const auto load = [&](int p0) {
+    // A chunk is loaded while the previous one is multiplied; in the launches that factorise blocks, whose tiles are few
+    // and wait on memory, while the one before the previous is (K = 64, a panel step's update, waits once). The others
+    // keep the registers for a third wave per SIMD.
+    constexpr int AHEAD = FUSE ? 2 : 1;
+    T ra[AHEAD][PER], rb[AHEAD][PER], rd[AHEAD][PER];
+    const auto load = [&](int p0, int to) {
 #pragma unroll
         for (int u = 0; u < PER; ++u)
         {
             const int64_t pp = min(p0 + kq + 4 * u, t.k - 1);
-            ra[u] = Ar[pp * ld];
-            rb[u] = Br[pp * ldb];
-            rd[u] = solve || PLAIN ? T(1) : dv[pp * (ld + 1)];
+            ra[to][u] = Ar[pp * ld];
+            rb[to][u] = Br[pp * ldb];
+            rd[to][u] = solve || PLAIN ? T(1) : dv[pp * (ld + 1)];
         }
     };
-    load(0);
-    for (int p0 = 0; p0 < t.k; p0 += TILE_K)
-    {
+    const auto multiply = [&](int p0, int from) {
         __syncthreads(); // the previous chunk's products have read the LDS
 #pragma unroll
         for (int u = 0; u < PER; ++u)
         {
             const int kk = kq + 4 * u;
             const bool term = p0 + kk < t.k;
-            const T av = pinned(ra[u]), bv = pinned(rb[u]), dd = pinned(rd[u]);
+            const T av = pinned(ra[from][u]), bv = pinned(rb[from][u]), dd = pinned(rd[from][u]);
             As[kk][row] = term && row < t.m ? (solve ? av : -av) : T(0);
             Bs[kk][row] = term && row < t.n ? (solve || PLAIN ? bv : bv * dd) : T(0);
         }
         __syncthreads();
-        if (p0 + TILE_K < t.k)
-            load(p0 + TILE_K);
+        if (p0 + AHEAD * TILE_K < t.k)
+            load(p0 + AHEAD * TILE_K, from);
 #pragma unroll
         for (int kk = 0; kk < TILE_K; kk += 4)
         {
@@ -729,6 +985,15 @@ __global__ __launch_bounds__(256, FUSE ? 2 : 1) void updateTilesKernel(DevicePla
                 for (int b = 0; b < 2; ++b)
                     acc[a][b] = Mfma<T>::step(av[a], bv[b], acc[a][b]);
         }
+    };
+    load(0, 0);
+    if (AHEAD == 2 && t.k > TILE_K)
+        load(TILE_K, AHEAD - 1);
+    for (int p0 = 0; p0 < t.k; p0 += AHEAD * TILE_K)
+    {
+        multiply(p0, 0);
+        if (AHEAD == 2 && p0 + TILE_K < t.k)
+            multiply(p0 + TILE_K, AHEAD - 1);
     }
     if (FUSE && t.mode == 2)
     {
@@ -736,8 +1001,9 @@ __global__ __launch_bounds__(256, FUSE ? 2 : 1) void updateTilesKernel(DevicePla
         constexpr int LD = TILE + 1;
         const int kb = t.colBase;
         __syncthreads(); // the products have read the LDS
-        for (int idx = tid; idx < TILE * LD; idx += 256)
-            lds[idx] = T(idx / LD == idx % LD ? 1 : 0);
+#pragma unroll
+        for (int q = 0; q < TILE / 4; ++q)
+            lds[(kq + 4 * q) * LD + row] = T(row == kq + 4 * q ? 1 : 0);
         __syncthreads();
 #pragma unroll
         for (int a = 0; a < 2; ++a)
@@ -754,7 +1020,7 @@ __global__ __launch_bounds__(256, FUSE ? 2 : 1) void updateTilesKernel(DevicePla
                         C[i + int64_t(j) * t.ldc] = acc[a][b][v]; // rows below a partial block: updated as usual
                 }
         __syncthreads();
-        factorBlockInLds(lds, p, t.supernode, t.rowBase, kb, panels, linv, diagOut, zeroAt);
+        factorBlockInLds(lds, kb, t.rowBase, int(t.ld), C, linv + t.ldb, diagOut + t.items, zeroAt + t.supernode);
         return;
     }
 #pragma unroll
@@ -2986,14 +3252,12 @@ hipError_t launchAssembly(const DevicePlan& p, const DeviceMatrix& a, T* panels,
 }
 
 template <typename T>
-hipError_t launchDiagonalBlocks(const DevicePlan& p, T* panels, T* linv, const int32_t* fronts, int frontCount, int k0,
-                                double* diagOut, int32_t* zeroAt, hipStream_t stream)
+hipError_t launchDiagonalBlocks(T* panels, T* linv, const DiagonalBlock* blocks, int count, double* diagOut,
+                                int32_t* zeroAt, hipStream_t stream)
 {
-    if (frontCount == 0)
+    if (count == 0)
         return hipSuccess;
-    // One wave per block: its barriers cost next to nothing.
-    hipLaunchKernelGGL(diagonalBlockKernel<T>, dim3(frontCount), dim3(256), 0, stream, p, panels, linv, fronts, k0,
-                       diagOut, zeroAt);
+    hipLaunchKernelGGL(diagonalBlockKernel<T>, dim3(count), dim3(256), 0, stream, panels, linv, blocks, diagOut, zeroAt);
     return hipGetLastError();
 }
 
@@ -3828,8 +4092,7 @@ hipError_t launchMfmaProbe(const double* a, const double* b, double* d, const fl
                                              int, double*, int32_t*, hipStream_t);                                     \
     template hipError_t launchAssembly<T>(const DevicePlan&, const DeviceMatrix&, T*, T*, const AssemblyBlock*,        \
                                           const AssemblyItem*, int, hipStream_t);                                      \
-    template hipError_t launchDiagonalBlocks<T>(const DevicePlan&, T*, T*, const int32_t*, int, int, double*,          \
-                                                int32_t*, hipStream_t);                                                \
+    template hipError_t launchDiagonalBlocks<T>(T*, T*, const DiagonalBlock*, int, double*, int32_t*, hipStream_t);     \
     template hipError_t launchUpdateTiles<T>(const DevicePlan&, T*, T*, T*, const UpdateTile*, int, double*, int32_t*, \
                                              bool, hipStream_t);                                                       \
     template hipError_t launchExtendTiles<T>(const DevicePlan&, T*, T*, const UpdateTile*, int, const int32_t*,        \

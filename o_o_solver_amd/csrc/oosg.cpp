@@ -452,7 +452,8 @@ struct oosg_plan
     double flops = 0.0;
 
     std::vector<Launch> schedule;
-    std::vector<int32_t> smallList, stepFronts;
+    std::vector<int32_t> smallList;
+    std::vector<oosg::DiagonalBlock> diagonalBlocks; // of the levels' first panel steps
     std::vector<oosg::AssemblyBlock> blocks;
     std::vector<oosg::AssemblyItem> items;
     std::vector<oosg::UpdateTile> tiles, bigTiles;
@@ -475,7 +476,7 @@ struct oosg_plan
     DeviceBuffer dTrailingBlocks, dTrailingItems, dTrailingPullStart, dTrailingPulls;
     // A mixed factor's boundary update matrices staged for their widening, and the ranges of that copy.
     DeviceBuffer widenTemp, widenRanges;
-    DeviceBuffer dSmallList, dStepFronts, dBlocks, dItems, dTiles, dBigTiles, dItemStarts, dExtendItems, dLevelList, dForwardTiles, dBackwardBlocks,
+    DeviceBuffer dSmallList, dDiagonalBlocks, dBlocks, dItems, dTiles, dBigTiles, dItemStarts, dExtendItems, dLevelList, dForwardTiles, dBackwardBlocks,
         dForwardSubtractions, dBackwardSubtractions,
         dForwardTriangles, dBackwardTriangles, dForwardTriangleSums, dBackwardTriangleSums, dInverseItems;
     oosg::DevicePlan dp{};
@@ -1573,7 +1574,7 @@ void buildSchedule(oosg_plan& p)
         {
             Launch diagonal{LaunchKind::Diagonal, PROFILE_DIAGONAL};
             diagonal.k0 = k0;
-            diagonal.offset = static_cast<int64_t>(p.stepFronts.size());
+            diagonal.offset = static_cast<int64_t>(p.diagonalBlocks.size());
             Launch solve{LaunchKind::Tiles, PROFILE_PANEL_SOLVE};
             solve.offset = static_cast<int64_t>(p.tiles.size());
             for (const int32_t s : large)
@@ -1582,7 +1583,10 @@ void buildSchedule(oosg_plan& p)
                 if (c <= k0)
                     continue;
                 const int kb = std::min(PANEL_BLOCK, c - k0), k1 = k0 + kb;
-                p.stepFronts.push_back(s);
+                // From the second step on, the previous step's update factorises the diagonal blocks.
+                if (k0 == 0)
+                    p.diagonalBlocks.push_back(
+                        oosg::DiagonalBlock{p.panelOff[s], p.linvOff[s], n, kb, p.first[s], s});
                 diagonal.flops += frontFlops(kb, 0);
                 // L(rows, blk) = F(rows, blk)·L11⁻ᵀ·D⁻¹: one mode-1 tile per 64 rows below the block.
                 for (int row = k1; row < n; row += 64)
@@ -1644,6 +1648,8 @@ void buildSchedule(oosg_plan& p)
                                 t.supernode = s;
                                 t.rowBase = J0;
                                 t.colBase = std::min(PANEL_BLOCK, c - J0);
+                                t.ldb = p.linvOff[s] + int64_t(J0) * PANEL_BLOCK;
+                                t.items = p.first[s] + J0;
                                 update.flops += frontFlops(t.colBase, 0);
                                 update.fuses = true;
                                 update.profile = PROFILE_PANEL_UPDATE_FUSED;
@@ -1662,7 +1668,7 @@ void buildSchedule(oosg_plan& p)
                 addUpdates(next, super1, super1 + SUPER_BLOCK, super0, super1, super1);
                 addUpdates(rest, super1 + SUPER_BLOCK, INT32_MAX, super0, super1, -1);
             }
-            diagonal.count = static_cast<int>(p.stepFronts.size() - diagonal.offset);
+            diagonal.count = static_cast<int>(p.diagonalBlocks.size() - diagonal.offset);
             diagonal.lane = solve.lane = inner.lane = next.lane = LANE_CRITICAL;
             const bool records = rest.count > 0 || k0 + PANEL_BLOCK >= maxC ||
                                  (k0 / PANEL_BLOCK) % SOLVED_RECORD_STEPS == SOLVED_RECORD_STEPS - 1;
@@ -1852,7 +1858,7 @@ void uploadPlan(oosg_plan& p)
     uploadSweepPlan(p);
     const hipStream_t st = p.stream;
     p.dSmallList = upload(p.smallList, st, "plan: small fronts");
-    p.dStepFronts = upload(p.stepFronts, st, "plan: panel step fronts");
+    p.dDiagonalBlocks = upload(p.diagonalBlocks, st, "plan: diagonal blocks");
     p.dBlocks = upload(p.blocks, st, "plan: assembly blocks");
     p.dItems = upload(p.items, st, "plan: assembly items");
     p.dTiles = upload(p.tiles, st, "plan: update tiles");
@@ -1870,8 +1876,7 @@ void uploadPlan(oosg_plan& p)
 // The plan's own arrays on the device (structure, launch lists), in bytes.
 uint64_t structureBytes(const oosg_plan& p)
 {
-    return (p.first.size() * 3 + p.rows.size() * 2 + p.children.size() + p.smallList.size() + p.stepFronts.size() +
-            p.levelList.size() * 2 + p.mediumList.size() + p.pullBase.size() + p.pulls.size() + p.gatherStart.size() +
+    return (p.first.size() * 3 + p.rows.size() * 2 + p.children.size() + p.smallList.size() + p.levelList.size() * 2 + p.mediumList.size() + p.pullBase.size() + p.pulls.size() + p.gatherStart.size() +
             p.gatherRows.size() + p.otherPosStart.size() * 2 + p.gatherChunks.size() * 8) *
                4 +
            p.panelOff.size() * 24 +
@@ -1879,7 +1884,7 @@ uint64_t structureBytes(const oosg_plan& p)
             p.backwardSubtractions.size()) *
                16 +
            (p.forwardTriangles.size() + p.backwardTriangles.size() + 2 * p.forwardTriangleSums.size()) * 16 +
-           p.inverseItems.size() * 8 + p.blocks.size() * sizeof(oosg::AssemblyBlock) +
+           p.inverseItems.size() * 8 + p.diagonalBlocks.size() * sizeof(oosg::DiagonalBlock) + p.blocks.size() * sizeof(oosg::AssemblyBlock) +
            p.items.size() * sizeof(oosg::AssemblyItem) +
            (p.tiles.size() + p.bigTiles.size()) * sizeof(oosg::UpdateTile) + p.itemStarts.size() * 4 +
            p.extendItems.size() * sizeof(oosg::AssemblyItem) +
@@ -1954,7 +1959,7 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
                          scaled ? m.dScale.as<double>() : nullptr};
     T* updates = p.updates.as<T>();
     const int32_t* smallList = p.dSmallList.as<int32_t>();
-    const int32_t* stepFronts = p.dStepFronts.as<int32_t>();
+    const oosg::DiagonalBlock* diagonalBlocks = p.dDiagonalBlocks.as<oosg::DiagonalBlock>();
     const oosg::AssemblyBlock* blocks = p.dBlocks.as<oosg::AssemblyBlock>();
     const oosg::AssemblyItem* items = p.dItems.as<oosg::AssemblyItem>();
     const int2* inverseItems = p.dInverseItems.as<int2>();
@@ -2078,8 +2083,7 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
                   "factor: assembly");
             break;
         case LaunchKind::Diagonal:
-            check(oosg::launchDiagonalBlocks<T>(p.dp, panels, linv, stepFronts + l.offset, l.count, l.k0, diagOut,
-                                                zeroAt, ls),
+            check(oosg::launchDiagonalBlocks<T>(panels, linv, diagonalBlocks + l.offset, l.count, diagOut, zeroAt, ls),
                   "factor: diagonal blocks");
             break;
         case LaunchKind::Tiles:
