@@ -201,11 +201,11 @@ hipError_t launchAssembly(const DevicePlan& p, const DeviceMatrix& a, T* panels,
 template <typename T>
 hipError_t launchDiagonalBlocks(T* panels, T* linv, const DiagonalBlock* blocks, int count, double* diagOut,
                                 int32_t* zeroAt, hipStream_t stream);
-// A step of the whole inverses X = L_FF⁻¹ of the wide supernodes' triangles (items (s, I << 16 | J)): step K >= 0
-// updates T_IJ = −Σ_{K'<=K} L_IK'·X_K'J for I > K >= J; step −1 sets X_IJ = L_II⁻¹·T_IJ (I > J) and X_II = L_II⁻¹.
+// A product of the whole inverses X = L_FF⁻¹ of the wide supernodes' triangles, on items {s, I << 16 | J, mid}: `which` 0
+// T_IJ = Σ_{J<=K<mid} L_IK·X_KJ (or X_II, the diagonal block's inverse, for I = J), 1 X_IJ = −Σ_{mid<=K<=I} X_IK·T_KJ.
 template <typename T>
-hipError_t launchTriangleInverse(const DevicePlan& p, const T* panels, T* linv, const int2* items, int count, int step,
-                                 hipStream_t stream);
+hipError_t launchTriangleInverse(const DevicePlan& p, const T* panels, T* linv, const int4* items, int count,
+                                 int which, hipStream_t stream);
 // The triangles of the wide supernodes in a sweep: items int4 {s, I, chunk, slot} write into their slot of partial
 // sums the chunk's part (SWEEP_CHUNK blocks J) of Σ_{J<=I} X_IJ·X(block J) (forward) or Σ_{J>=I} X_JIᵀ·X(block J)
 // (transpose); the subtraction launch's items with bit 29 (assign) then set X's rows of block I to the sum.

@@ -1198,167 +1198,103 @@ __global__ __launch_bounds__(256) void extendTilesKernel(DevicePlan p, T* panels
 
 // ---- whole inverses of the wide supernodes' triangles -----------------------------------------------------------
 //
-// X = L_FF⁻¹ (c × c, leading dimension c) by blocks of 64, right-looking: with T_IJ = −Σ_{K<I} L_IK·X_KJ (I > J), X_IJ =
-// L_II⁻¹·T_IJ. Step K (one launch) takes the items (s, I, J), I > K >= J: T_IJ = −L_IK·X_KJ (J = K, X_KK = L_KK⁻¹) or
-// T_IJ −= L_IK·X_KJ (J < K), where X_KJ = L_KK⁻¹·T_KJ is formed in the workgroup from T_KJ (final since step K − 1; no
-// item of step K writes row block K). The last launch (items (s, I, J), I >= J) sets X_IJ = L_II⁻¹·T_IJ in place, or
-// X_II = L_II⁻¹ from the diagonal block's inverse. Blocks other than the last are full (64), so only row block I can
-// be narrower (ib). Four waves of 32 × 32 over a 64 × 64 tile, 16 × 16 × 4 MFMA blocks; products of 64 terms staged
-// through LDS in chunks of 32.
-
-// The operands of a product of 64 terms for a 64 × 64 tile, held in registers: a thread stages 16 values of A(i, t)
-// (row i = tid mod 64, terms kq + 4u of each half) and 16 of B(t, j) (term bk of each half, columns bj + 8u). All of
-// an item's operands are loaded before its first product, so its global loads wait once, not once per chunk.
-template <typename T> struct TileTerms
+// X = L_FF⁻¹ (c × c, leading dimension c) by halving its column blocks of 64: the inverse of [L_11 0; L_21 L_22] has
+// X_21 = −X_22·L_21·X_11, so a node of the halvings, its halves inverted, takes two products: T = L_21·X_11 (SECOND false)
+// and X_21 = −X_22·T. T lies transposed in X's upper triangle, T_IJ where block (J, I) of X would be, which nothing else
+// uses. All the nodes of a height (and of many supernodes) go in one launch per product: 2·⌈log2 of the blocks⌉ launches,
+// against one or two per column block for a right-looking inverse, whose few items each (8.7 µs a launch, 66 of them in
+// the 137 × 91 plate's factor: 0.57 of 3.4 ms) waited for each other. Blocks other than the last are full (64), so only
+// row block I can be narrower (ib).
+//
+// One 64 × 64 tile per workgroup, four waves of 32 × 32 in 16 × 16 × 4 MFMA blocks; the 64 terms of a block K go through
+// LDS at once, the next block's loaded into registers meanwhile. Items int4 {s, I << 16 | J, mid}: the columns' halves
+// meet at block mid; I = J copies the diagonal block's inverse.
+template <typename T, bool SECOND>
+__global__ __launch_bounds__(256) void triangleInverseKernel(DevicePlan p, const T* panels, T* linv, const int4* items)
 {
-    T a[16], b[16];
-};
-
-// Loads A(i, t) = a(i, t) for i < rowsA and B(t, j) = b(t, j) for t < terms; a and b are given positions clamped into
-// range, and the values beyond are zeroed when staged.
-template <typename T, typename FA, typename FB>
-__device__ inline void loadTileTerms(TileTerms<T>& s, int rowsA, int terms, FA a, FB b)
-{
-    const int tid = threadIdx.x;
-    const int row = tid & (TILE - 1), kq = tid >> 6;
-    const int bk = tid & 31, bj = tid >> 5;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-    {
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            s.a[8 * h + u] = a(min(row, rowsA - 1), min(32 * h + kq + 4 * u, terms - 1));
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            s.b[8 * h + u] = b(min(32 * h + bk, terms - 1), bj + 8 * u);
-    }
-}
-
-// acc += A·B over the staged terms, through LDS in two chunks of 32. Four waves of 32 × 32 over the tile, 16 × 16 × 4
-// MFMA blocks.
-template <typename T>
-__device__ inline void multiplyTileTerms(typename Mfma<T>::Acc (&acc)[2][2], T (*As)[TILE + 4], T (*Bs)[TILE + 4],
-                                         const TileTerms<T>& s, int rowsA, int terms)
-{
+    __shared__ T As[TILE][TILE + 4];
+    __shared__ T Bs[TILE][TILE + 4];
+    constexpr int PER = TILE * TILE / 256;
+    const int4 item = items[blockIdx.x];
+    const int s = item.x, I = item.y >> 16, J = item.y & 0xFFFF, mid = item.z;
+    const int c = p.ncol[s], n = c + p.nrow[s];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     const int row = tid & (TILE - 1), kq = tid >> 6;
-    const int bk = tid & 31, bj = tid >> 5;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+    const T* inverses = linv + p.linvOff[s];
+    T* X = linv + p.linvOff[s] + blockInverseValues(c);
+    const int i0 = TILE * I, j0 = TILE * J, ib = min(TILE, c - i0);
+    if (I == J)
     {
-        __syncthreads(); // the previous chunk's products have read the LDS
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            As[kq + 4 * u][row] = row < rowsA && 32 * h + kq + 4 * u < terms ? pinned(s.a[8 * h + u]) : T(0);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            Bs[bk][bj + 8 * u] = 32 * h + bk < terms ? pinned(s.b[8 * h + u]) : T(0);
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 32; kk += 4)
-        {
-            const int ka = kk + (lane >> 4);
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y)
-                    acc[x][y] = Mfma<T>::step(As[ka][wm + x * 16 + (lane & 15)], Bs[ka][wn + y * 16 + (lane & 15)],
-                                              acc[x][y]);
-        }
+        const T* inv = inverses + int64_t(i0) * TILE; // ib × ib, leading dimension ib
+        for (int j = wave; j < ib; j += 4)
+            if (lane < ib)
+                X[(i0 + lane) + int64_t(i0 + j) * c] = inv[lane + j * ib];
+        return;
     }
-}
-
-template <typename T> __device__ inline void zeroTile(typename Mfma<T>::Acc (&acc)[2][2])
-{
+    const T* L = panels + p.panelOff[s];
+    const int first = SECOND ? mid : J, last = SECOND ? I : mid - 1;
+    T ra[PER], rb[PER];
+    // A(i, t): row i = tid mod 64, terms t = kq + 4u. B(t, j): the first product's X_KJ with t = tid mod 64, columns
+    // kq + 4u; the second's T_KJ, transposed in memory, with j = tid mod 64, terms kq + 4u.
+    const auto load = [&](int K) {
+        const int k0 = TILE * K, terms = min(TILE, c - k0);
+        const bool diagonalA = SECOND && K == I, diagonalB = !SECOND && K == J;
+        const T* A = SECOND ? (diagonalA ? inverses + int64_t(i0) * TILE : X + i0 + int64_t(k0) * c)
+                            : L + i0 + int64_t(k0) * n;
+        const int64_t lda = SECOND ? (diagonalA ? ib : c) : n;
+        const T* B = SECOND ? X + j0 + int64_t(k0) * c
+                            : (diagonalB ? inverses + int64_t(k0) * TILE : X + k0 + int64_t(j0) * c);
+        const int64_t ldb = diagonalB ? TILE : c;
+        const int rowA = min(row, ib - 1);
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+        {
+            const int q = kq + 4 * u;
+            ra[u] = A[rowA + min(q, terms - 1) * lda];
+            rb[u] = B[row + (SECOND ? min(q, terms - 1) : q) * ldb]; // the first product's K is a full block
+        }
+    };
+    typename Mfma<T>::Acc acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y)
             acc[x][y] = typename Mfma<T>::Acc{0, 0, 0, 0};
-}
-
-// The element (i, j) of the tile that acc[x][y][v] holds on this lane.
-__device__ inline int tileRow(int x, int v, int lane, int wave, bool fp64)
-{
-    return (wave >> 1) * 32 + x * 16 + (fp64 ? (lane >> 4) + 4 * v : 4 * (lane >> 4) + v);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void triangleInverseKernel(DevicePlan p, const T* panels, T* linv, const int2* items,
-                                                             int step)
-{
-    __shared__ T As[32][TILE + 4];
-    __shared__ T Bs[32][TILE + 4];
-    const int2 item = items[blockIdx.x];
-    const int s = item.x, I = item.y >> 16, J = item.y & 0xFFFF;
-    const int c = p.ncol[s], n = c + p.nrow[s];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wn = (wave & 1) * 32;
-    T* X = linv + p.linvOff[s] + blockInverseValues(c);
-    const int i0 = TILE * I, j0 = TILE * J, ib = min(TILE, c - i0);
-    const bool fp64 = sizeof(T) == 8;
-    typename Mfma<T>::Acc acc[2][2];
-    if (step < 0)
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    load(first);
+    for (int K = first; K <= last; ++K)
     {
-        // A row block's final values: X_II from the diagonal block's inverse, or X_IJ = L_II⁻¹·T_IJ (T_IJ complete:
-        // before step I, or in the last launch).
-        const T* inv = linv + p.linvOff[s] + int64_t(i0) * TILE; // ib × ib, leading dimension ib
-        if (I == J)
+        const int terms = min(TILE, c - TILE * K);
+        __syncthreads(); // the previous block's products have read the LDS
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
         {
-            for (int j = wave; j < ib; j += 4)
-                if (lane < ib)
-                    X[(i0 + lane) + int64_t(i0 + j) * c] = inv[lane + j * ib];
-            return;
+            const int q = kq + 4 * u;
+            const T av = pinned(ra[u]), bv = pinned(rb[u]);
+            As[q][row] = row < ib && q < terms ? av : T(0);
+            Bs[q][row] = !SECOND || q < terms ? bv : T(0); // [column][term] for the first product, [term][column]
         }
-        TileTerms<T> terms;
-        loadTileTerms<T>(terms, ib, ib, [&](int i, int t) { return inv[i + t * ib]; },
-                         [&](int t, int j) { return X[(i0 + t) + int64_t(j0 + j) * c]; });
-        zeroTile<T>(acc);
-        multiplyTileTerms<T>(acc, As, Bs, terms, ib, ib);
-        __syncthreads(); // every wave has read T_IJ before any writes X_IJ over it
-    }
-    else
-    {
-        // The terms of steps K0 .. K, in that order (K0 = K − 1 for a paired step, flag bit 16: step K − 1 did only
-        // the items of row block K): T_IJ −= L_I,Kt·X_Kt,J for J < Kt (row block Kt is final before step Kt), or
-        // T_IKt = −L_I,Kt·L_KtKt⁻¹ for J = Kt. The accumulators start from T_IJ (J < K0) or zero, L enters negated.
-        const int K = step & 0xFFFF, K0 = ((step >> 16) & 1) ? K - 1 : K;
-        const T* L = panels + p.panelOff[s];
-        if (J < K0)
+        __syncthreads();
+        if (K < last)
+            load(K + 1);
+#pragma unroll
+        for (int kk = 0; kk < TILE; kk += 4)
         {
+            const int ka = kk + (lane >> 4);
+            T av[2], bv[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+            {
+                const int j = wn + x * 16 + (lane & 15);
+                av[x] = As[ka][wm + x * 16 + (lane & 15)];
+                bv[x] = SECOND ? Bs[ka][j] : Bs[j][ka];
+            }
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
                 for (int y = 0; y < 2; ++y)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        acc[x][y][v] = X[(i0 + min(tileRow(x, v, lane, wave, fp64), ib - 1)) +
-                                         int64_t(j0 + wn + y * 16 + (lane & 15)) * c];
+                    acc[x][y] = Mfma<T>::step(av[x], bv[y], acc[x][y]);
         }
-        else
-            zeroTile<T>(acc);
-        // The operands of both steps are loaded before the first product (step Kt has a term when J <= Kt; J <= K).
-        TileTerms<T> terms[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-        {
-            const int Kt = K0 + e;
-            if (Kt > K || J > Kt)
-                continue; // the same for the whole workgroup
-            const int kt0 = TILE * Kt;
-            const T* invKt = linv + p.linvOff[s] + int64_t(kt0) * TILE; // 64 × 64 (block Kt is full)
-            if (J < Kt)
-                loadTileTerms<T>(terms[e], ib, TILE, [&](int i, int t) { return -L[(i0 + i) + int64_t(kt0 + t) * n]; },
-                                 [&](int t, int j) { return X[(kt0 + t) + int64_t(j0 + j) * c]; });
-            else
-                loadTileTerms<T>(terms[e], ib, TILE, [&](int i, int t) { return -L[(i0 + i) + int64_t(kt0 + t) * n]; },
-                                 [&](int t, int j) { return invKt[t + j * TILE]; });
-        }
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-            if (K0 + e <= K && J <= K0 + e)
-                multiplyTileTerms<T>(acc, As, Bs, terms[e], ib, TILE);
     }
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -1367,9 +1303,13 @@ __global__ __launch_bounds__(256) void triangleInverseKernel(DevicePlan p, const
 #pragma unroll
             for (int v = 0; v < 4; ++v)
             {
-                const int i = tileRow(x, v, lane, wave, fp64), j = wn + y * 16 + (lane & 15);
-                if (i < ib)
-                    X[(i0 + i) + int64_t(j0 + j) * c] = acc[x][y][v];
+                const int i = wm + x * 16 + Mfma<T>::row(lane, v), j = wn + y * 16 + (lane & 15);
+                if (i >= ib)
+                    continue;
+                if (SECOND)
+                    X[(i0 + i) + int64_t(j0 + j) * c] = -acc[x][y][v];
+                else
+                    X[(j0 + j) + int64_t(i0 + i) * c] = acc[x][y][v];
             }
 }
 
@@ -3417,11 +3357,15 @@ hipError_t launchBackward(const DevicePlan& p, const TP* panels, const TP* linv,
 }
 
 template <typename T>
-hipError_t launchTriangleInverse(const DevicePlan& p, const T* panels, T* linv, const int2* items, int count, int step,
-                                 hipStream_t stream)
+hipError_t launchTriangleInverse(const DevicePlan& p, const T* panels, T* linv, const int4* items, int count,
+                                 int which, hipStream_t stream)
 {
-    if (count > 0)
-        hipLaunchKernelGGL(triangleInverseKernel<T>, dim3(count), dim3(256), 0, stream, p, panels, linv, items, step);
+    if (count == 0)
+        return hipSuccess;
+    if (which == 0)
+        hipLaunchKernelGGL((triangleInverseKernel<T, false>), dim3(count), dim3(256), 0, stream, p, panels, linv, items);
+    else
+        hipLaunchKernelGGL((triangleInverseKernel<T, true>), dim3(count), dim3(256), 0, stream, p, panels, linv, items);
     return hipGetLastError();
 }
 
@@ -4109,7 +4053,7 @@ hipError_t launchMfmaProbe(const double* a, const double* b, double* d, const fl
                                              const int32_t*, int, hipStream_t);                                        \
     template hipError_t launchTinyBackward<T>(const DevicePlan&, const T*, const T*, double*, int, const int32_t*, int, \
                                               hipStream_t);                                                            \
-    template hipError_t launchTriangleInverse<T>(const DevicePlan&, const T*, T*, const int2*, int, int, hipStream_t); \
+    template hipError_t launchTriangleInverse<T>(const DevicePlan&, const T*, T*, const int4*, int, int, hipStream_t); \
     template hipError_t launchTriangleProducts<T>(const DevicePlan&, const T*, const double*, int, const int4*, int,   \
                                                   int, double*, hipStream_t);                                          \
     template size_t smallFrontBytes<T>(int);

@@ -436,17 +436,18 @@ struct oosg_plan
     std::vector<int64_t> forwardTriangleStart, backwardTriangleStart, triangleSumStart;
     struct InverseRound
     {
-        int step; // −1: the last launch
-        int64_t offset;
-        int count;
-        double flops;
-        // Before step K: row block K's final values (items (s, K, J < K), launched as step −1).
-        int64_t rowOffset = 0;
-        int rowCount = 0;
-        double rowFlops = 0.0;
+        int ready = 0; // the column blocks whose panel solve it waits for
+        // The items of T = L_21·X_11 (with the copies of the diagonal blocks) and of X_21 = −X_22·T, which do not
+        // depend on each other within a round.
+        int64_t offset[2] = {0, 0};
+        int count[2] = {0, 0};
+        double flops[2] = {0.0, 0.0};
     };
-    std::vector<int2> inverseItems;
+    std::vector<int4> inverseItems;
+    // By level, for the streams beside the critical path; and all levels' together, for one stream after the last
+    // level (a round per height of the halvings: the first product's launch, then the second's).
     std::vector<std::vector<InverseRound>> inverseRounds;
+    std::vector<InverseRound> mergedInverses;
     int32_t levels = 0;
     int64_t smallFronts = 0, largeFronts = 0;
     double flops = 0.0;
@@ -754,6 +755,9 @@ void pollCancellation(oosg_plan& p)
 }
 
 // ---- plan --------------------------------------------------------------------------------------------------------
+
+// The column blocks solved between two rounds of the whole inverses beside a level's panel steps.
+constexpr int INVERSE_BLOCKS = 8;
 
 void deriveLevels(oosg_plan& p);
 oosg_status createPlan(const oosg_symbolic_desc* symbolic, int32_t trailing_dof_count, bool outOfCore, int32_t device,
@@ -1105,6 +1109,136 @@ void windowLayout(oosg_plan& p, const std::vector<int32_t>& height)
 
 // From the structure (first, ncol, nrow, parent, children): the offsets of the panels, update matrices and inverses,
 // the levels by height, the flops, and the sweeps' work lists by level.
+// The halvings of a wide triangle's column blocks: node [a, b) with its middle, the nodes of its halves (-1: a single
+// block, whose inverse the factorisation gives) and its height. Children come before their parents.
+struct Halving
+{
+    int a, mid, b, left, right, height;
+};
+
+int halve(std::vector<Halving>& nodes, int a, int b)
+{
+    if (b - a == 1)
+        return -1;
+    const int mid = a + (b - a + 1) / 2;
+    const int left = halve(nodes, a, mid), right = halve(nodes, mid, b);
+    const int height = 1 + std::max(left < 0 ? 0 : nodes[left].height, right < 0 ? 0 : nodes[right].height);
+    nodes.push_back(Halving{a, mid, b, left, right, height});
+    return static_cast<int>(nodes.size()) - 1;
+}
+
+// The items of one product of a node of supernode s: T = L_21·X_11 (which 0) or X_21 = −X_22·T (1), a block (I, J) of
+// 64 × 64 each.
+void addInverseItems(oosg_plan& p, oosg_plan::InverseRound& round, int32_t s, const Halving& node, int which)
+{
+    for (int I = node.mid; I < node.b; ++I)
+        for (int J = node.a; J < node.mid; ++J)
+        {
+            p.inverseItems.push_back(make_int4(s, (I << 16) | J, node.mid, 0));
+            round.flops[which] += 2.0 * 64.0 * 64.0 * 64.0 * (which == 0 ? node.mid - J : I - node.mid + 1);
+        }
+}
+
+void addDiagonalInverseItems(oosg_plan& p, int32_t s)
+{
+    for (int I = 0; I < (p.ncol[s] + 63) / 64; ++I)
+        p.inverseItems.push_back(make_int4(s, (I << 16) | I, 0, 0));
+}
+
+// The rounds of a level's whole inverses for a stream beside the critical path: at every INVERSE_BLOCKS column blocks
+// whose panel solve is done, and at the level's end, the products whose operands are there, round by round.
+std::vector<oosg_plan::InverseRound> levelInverseRounds(oosg_plan& p, int32_t l, int maxBlocks)
+{
+    std::vector<oosg_plan::InverseRound> rounds;
+    struct Triangle
+    {
+        int32_t s;
+        std::vector<Halving> nodes;
+        std::vector<char> done; // 0 nothing, 1 T, 2 X_21
+    };
+    std::vector<Triangle> triangles;
+    for (int32_t q = p.levelStart[l]; q < p.levelStart[l + 1]; ++q)
+    {
+        const int32_t s = p.levelList[q];
+        if (!oosg::keepsTriangleInverse(p.ncol[s]))
+            continue;
+        Triangle t{s, {}, {}};
+        halve(t.nodes, 0, (p.ncol[s] + 63) / 64);
+        t.done.assign(t.nodes.size(), 0);
+        triangles.push_back(std::move(t));
+    }
+    for (int ready = INVERSE_BLOCKS; !triangles.empty(); ready += INVERSE_BLOCKS)
+    {
+        const bool last = ready >= maxBlocks;
+        for (;;)
+        {
+            oosg_plan::InverseRound round;
+            round.ready = std::min(ready, maxBlocks);
+            std::vector<std::pair<char*, char>> reached;
+            for (int which = 0; which < 2; ++which)
+            {
+                round.offset[which] = static_cast<int64_t>(p.inverseItems.size());
+                for (Triangle& t : triangles)
+                    for (size_t k = 0; k < t.nodes.size(); ++k)
+                    {
+                        const Halving& node = t.nodes[k];
+                        const int child = which == 0 ? node.left : node.right;
+                        if (t.done[k] != which || (which == 0 ? node.mid : node.b) > ready ||
+                            (child >= 0 && t.done[child] != 2))
+                            continue;
+                        addInverseItems(p, round, t.s, node, which);
+                        reached.emplace_back(&t.done[k], static_cast<char>(which + 1));
+                    }
+                // The copies of the diagonal blocks, with the level's last first products.
+                if (which == 0 && last && (rounds.empty() || rounds.back().ready < maxBlocks))
+                    for (const Triangle& t : triangles)
+                        addDiagonalInverseItems(p, t.s);
+                round.count[which] = static_cast<int>(p.inverseItems.size() - round.offset[which]);
+            }
+            for (const auto& r : reached)
+                *r.first = r.second;
+            if (round.count[0] + round.count[1] == 0)
+                break;
+            rounds.push_back(round);
+        }
+        if (last)
+            break;
+    }
+    return rounds;
+}
+
+// The whole inverses of every level's wide triangles together.
+void mergeInverses(oosg_plan& p)
+{
+    p.mergedInverses.clear();
+    std::vector<std::pair<int32_t, std::vector<Halving>>> triangles;
+    int heights = 0;
+    for (const int32_t s : p.levelList)
+        if (oosg::keepsTriangleInverse(p.ncol[s]))
+        {
+            triangles.emplace_back(s, std::vector<Halving>());
+            halve(triangles.back().second, 0, (p.ncol[s] + 63) / 64);
+            heights = std::max(heights, triangles.back().second.back().height);
+        }
+    for (int h = 1; h <= heights; ++h)
+    {
+        oosg_plan::InverseRound round;
+        for (int which = 0; which < 2; ++which)
+        {
+            round.offset[which] = static_cast<int64_t>(p.inverseItems.size());
+            for (const auto& t : triangles)
+                for (const Halving& node : t.second)
+                    if (node.height == h)
+                        addInverseItems(p, round, t.first, node, which);
+            if (h == 1 && which == 0)
+                for (const auto& t : triangles)
+                    addDiagonalInverseItems(p, t.first);
+            round.count[which] = static_cast<int>(p.inverseItems.size() - round.offset[which]);
+        }
+        p.mergedInverses.push_back(round);
+    }
+}
+
 void deriveLevels(oosg_plan& p)
 {
     const int32_t S = p.S;
@@ -1286,47 +1420,9 @@ void deriveLevels(oosg_plan& p)
         p.forwardTriangleStart[l + 1] = static_cast<int64_t>(p.forwardTriangles.size());
         p.backwardTriangleStart[l + 1] = static_cast<int64_t>(p.backwardTriangles.size());
         p.triangleSumStart[l + 1] = static_cast<int64_t>(p.forwardTriangleSums.size());
-        std::vector<oosg_plan::InverseRound> rounds;
-        // Steps K = 0 .. maxBlocks − 2 (items (s, I, J), I > K >= J), each after row block K's final values (items
-        // (s, K, J < K), for 1 <= K <= blocks − 2), then the last launch (the diagonal blocks and the last row block,
-        // step −1).
-        constexpr double ITEM_FLOPS = 2.0 * 64.0 * 64.0 * 64.0;
-        for (int K = 0; K <= maxBlocks - 1; ++K)
-        {
-            const bool last = K == maxBlocks - 1;
-            oosg_plan::InverseRound round{last ? -1 : (K % 2 == 1 ? K | (1 << 16) : K), 0, 0, 0.0};
-            round.rowOffset = static_cast<int64_t>(p.inverseItems.size());
-            for (int32_t q = p.levelStart[l]; !last && K >= 1 && q < p.levelStart[l + 1]; ++q)
-            {
-                const int32_t s = p.levelList[q];
-                if (oosg::keepsTriangleInverse(p.ncol[s]) && K <= (p.ncol[s] + 63) / 64 - 2)
-                    for (int J = 0; J < K; ++J)
-                        p.inverseItems.push_back(make_int2(s, (K << 16) | J));
-            }
-            round.rowCount = static_cast<int>(p.inverseItems.size() - round.rowOffset);
-            round.rowFlops = round.rowCount * ITEM_FLOPS;
-            round.offset = static_cast<int64_t>(p.inverseItems.size());
-            for (int32_t q = p.levelStart[l]; q < p.levelStart[l + 1]; ++q)
-            {
-                const int32_t s = p.levelList[q];
-                const int blocks = (p.ncol[s] + 63) / 64;
-                if (!oosg::keepsTriangleInverse(p.ncol[s]))
-                    continue;
-                // Steps in pairs: an even step K does the items of row block K + 1 only, the odd step K + 1 every
-                // item below with the terms of both steps (each T_IJ read and written once for two steps).
-                for (int I = 0; I < blocks; ++I)
-                    for (int J = 0; J <= I; ++J)
-                        if (last ? (I == J || I == blocks - 1) : (K % 2 == 0 ? I == K + 1 && J <= K : I > K && J <= K))
-                        {
-                            p.inverseItems.push_back(make_int2(s, (I << 16) | J));
-                            round.flops += ITEM_FLOPS * (!last && K % 2 == 1 && J < K ? 2.0 : 1.0);
-                        }
-            }
-            round.count = static_cast<int>(p.inverseItems.size() - round.offset);
-            rounds.push_back(round);
-        }
-        p.inverseRounds.push_back(std::move(rounds));
+        p.inverseRounds.push_back(levelInverseRounds(p, l, maxBlocks));
     }
+    mergeInverses(p);
     placeUpdateMatrices(p, height);
     splitTinySupernodes(p);
     if (p.outOfCore)
@@ -1353,28 +1449,23 @@ Launch syncLaunch(int lane, int wait, int record)
 
 // A launch of one step of a level's whole inverses, on the inverses' stream after the event `wait`.
 // The launch of a step's row block finals (before the step's own launch).
-Launch inverseRowsLaunch(const oosg_plan::InverseRound& round, int wait)
+// The launches of a round of the whole inverses, the first after `wait`.
+void pushInverseRound(oosg_plan& p, const oosg_plan::InverseRound& round, int wait)
 {
-    Launch rows{LaunchKind::Inverse, PROFILE_TRIANGLE_INVERSES};
-    rows.offset = round.rowOffset;
-    rows.count = round.rowCount;
-    rows.k0 = -1;
-    rows.flops = round.rowFlops;
-    rows.lane = LANE_INVERSES;
-    rows.wait = wait;
-    return rows;
-}
-
-Launch inverseLaunch(const oosg_plan::InverseRound& round, int wait)
-{
-    Launch inverse{LaunchKind::Inverse, PROFILE_TRIANGLE_INVERSES};
-    inverse.offset = round.offset;
-    inverse.count = round.count;
-    inverse.k0 = round.step;
-    inverse.flops = round.flops;
-    inverse.lane = LANE_INVERSES;
-    inverse.wait = wait;
-    return inverse;
+    for (int which = 0; which < 2; ++which)
+    {
+        if (round.count[which] == 0)
+            continue;
+        Launch inverse{LaunchKind::Inverse, PROFILE_TRIANGLE_INVERSES};
+        inverse.offset = round.offset[which];
+        inverse.count = round.count[which];
+        inverse.k0 = which;
+        inverse.flops = round.flops[which];
+        inverse.lane = LANE_INVERSES;
+        inverse.wait = wait;
+        p.schedule.push_back(inverse);
+        wait = -1;
+    }
 }
 
 // The assembly blocks of the panel part (columns < c) of the front of s, each with the parts of its children's update
@@ -1462,8 +1553,6 @@ void buildSchedule(oosg_plan& p)
     using oosg::PANEL_BLOCK;
     // Columns of a super-block: the trailing update beyond it is one product with K = SUPER_BLOCK.
     constexpr int SUPER_BLOCK = 4 * PANEL_BLOCK;
-    // Panel steps between two records of EVENT_SOLVED (when the bulk update needs none sooner).
-    constexpr int SOLVED_RECORD_STEPS = 4;
     // Every event is recorded once on the critical stream first, so that each wait refers to a record of the same
     // sequence (a captured graph has no outside dependencies).
     p.schedule.push_back(syncLaunch(LANE_CRITICAL, -1, EVENT_SOLVED));
@@ -1556,20 +1645,7 @@ void buildSchedule(oosg_plan& p)
         p.schedule.push_back(assemble);
         // Panel steps.
         // A record of EVENT_SOLVED on the critical stream delays its next launch by several microseconds, so a step
-        // records only when the bulk update needs it, every SOLVED_RECORD_STEPS steps, and at the level's last step.
-        // pendingInverses: the whole inverses' steps whose panel solve is done but not yet recorded (they wait for
-        // the next record).
-        std::vector<size_t> pendingInverses;
-        const auto launchPendingInverses = [&]
-        {
-            for (const size_t K : pendingInverses)
-            {
-                if (p.inverseRounds[l][K].rowCount > 0)
-                    p.schedule.push_back(inverseRowsLaunch(p.inverseRounds[l][K], EVENT_SOLVED));
-                p.schedule.push_back(inverseLaunch(p.inverseRounds[l][K], EVENT_SOLVED));
-            }
-            pendingInverses.clear();
-        };
+        // records only when the bulk update or a round of the whole inverses needs it, and at the level's last step.
         for (int k0 = 0; k0 < maxC; k0 += PANEL_BLOCK)
         {
             Launch diagonal{LaunchKind::Diagonal, PROFILE_DIAGONAL};
@@ -1671,7 +1747,7 @@ void buildSchedule(oosg_plan& p)
             diagonal.count = static_cast<int>(p.diagonalBlocks.size() - diagonal.offset);
             diagonal.lane = solve.lane = inner.lane = next.lane = LANE_CRITICAL;
             const bool records = rest.count > 0 || k0 + PANEL_BLOCK >= maxC ||
-                                 (k0 / PANEL_BLOCK) % SOLVED_RECORD_STEPS == SOLVED_RECORD_STEPS - 1;
+                                 (k0 / PANEL_BLOCK + 1) % INVERSE_BLOCKS == 0;
             Launch& solvedAt = solve.count > 0 ? solve : diagonal;
             if (records)
                 solvedAt.record = EVENT_SOLVED;
@@ -1694,24 +1770,15 @@ void buildSchedule(oosg_plan& p)
                 rest.record = EVENT_RESTED;
                 p.schedule.push_back(rest);
             }
-            // Step K = k0 / 64 of the level's whole inverses reads the panels' column block K (rows below block K),
-            // final once this step's solve is done: it runs beside the next steps instead of after the level.
-            const size_t K = static_cast<size_t>(k0 / PANEL_BLOCK);
-            const std::vector<oosg_plan::InverseRound>& rounds = p.inverseRounds[l];
-            if (K + 1 < rounds.size() && rounds[K].count > 0)
-            {
-                if (solve.count == 0)
-                    throw std::logic_error("plan: an inverse step without a panel solve");
-                pendingInverses.push_back(K);
-            }
-            // A recorded step's solve covers the earlier steps' (one stream, in order).
-            if (records && (solve.count > 0 || k0 == 0))
-                launchPendingInverses();
-        }
-        if (!pendingInverses.empty())
-        {
-            p.schedule.push_back(syncLaunch(LANE_CRITICAL, -1, EVENT_SOLVED));
-            launchPendingInverses();
+            // The whole inverses' rounds whose panels this step completes run beside the next steps.
+            const int solvedBlocks = k0 / PANEL_BLOCK + 1;
+            bool waits = true;
+            for (const oosg_plan::InverseRound& round : p.inverseRounds[l])
+                if (round.ready == solvedBlocks && solvedBlocks % INVERSE_BLOCKS == 0 && k0 + PANEL_BLOCK < maxC)
+                {
+                    pushInverseRound(p, round, waits ? EVENT_SOLVED : -1);
+                    waits = false;
+                }
         }
         // The level's panels are final once the bulk stream is done with them.
         p.schedule.push_back(syncLaunch(LANE_CRITICAL, EVENT_RESTED, EVENT_PANELS));
@@ -1790,9 +1857,14 @@ void buildSchedule(oosg_plan& p)
             tilesLaunch.big[0] = tilesLaunch.big[1] = tilesLaunch.bigCount >= 2048;
             p.schedule.push_back(tilesLaunch);
         }
-        // The last launch of the level's whole inverses (X_IJ = L_II⁻¹·T_IJ), once its panels are final.
-        if (!p.inverseRounds[l].empty() && p.inverseRounds[l].back().count > 0)
-            p.schedule.push_back(inverseLaunch(p.inverseRounds[l].back(), EVENT_PANELS));
+        // The rest of the level's whole inverses, once its panels are final.
+        bool waits = true;
+        for (const oosg_plan::InverseRound& round : p.inverseRounds[l])
+            if (round.ready % INVERSE_BLOCKS != 0 || round.ready * PANEL_BLOCK >= maxC)
+            {
+                pushInverseRound(p, round, waits ? EVENT_PANELS : -1);
+                waits = false;
+            }
     }
     // The other streams join the critical one (each first waits for a record of this sequence, so that both belong to
     // it even when they had nothing to do).
@@ -1884,7 +1956,7 @@ uint64_t structureBytes(const oosg_plan& p)
             p.backwardSubtractions.size()) *
                16 +
            (p.forwardTriangles.size() + p.backwardTriangles.size() + 2 * p.forwardTriangleSums.size()) * 16 +
-           p.inverseItems.size() * 8 + p.diagonalBlocks.size() * sizeof(oosg::DiagonalBlock) + p.blocks.size() * sizeof(oosg::AssemblyBlock) +
+           p.inverseItems.size() * 16 + p.diagonalBlocks.size() * sizeof(oosg::DiagonalBlock) + p.blocks.size() * sizeof(oosg::AssemblyBlock) +
            p.items.size() * sizeof(oosg::AssemblyItem) +
            (p.tiles.size() + p.bigTiles.size()) * sizeof(oosg::UpdateTile) + p.itemStarts.size() * 4 +
            p.extendItems.size() * sizeof(oosg::AssemblyItem) +
@@ -1943,6 +2015,17 @@ template <typename TP>
 void forwardSweep(oosg_plan& p, const TP* panels, const TP* linv, int k, int32_t l0, int32_t l1, hipStream_t st);
 void ensureSolveBuffers(oosg_plan& p);
 
+// The whole inverses of every level, after its panels.
+template <typename T> void runMergedInverses(const oosg_plan& p, const T* panels, T* linv, hipStream_t st)
+{
+    for (const oosg_plan::InverseRound& round : p.mergedInverses)
+        for (int which = 0; which < 2; ++which)
+            check(oosg::launchTriangleInverse<T>(p.dp, panels, linv,
+                                                 p.dInverseItems.as<int4>() + round.offset[which], round.count[which],
+                                                 which, st),
+                  "factor: triangle inverses");
+}
+
 // cancellable: launched one launch at a time (not captured), so the cancellation is polled between levels.
 template <typename T>
 void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* diagOut, int32_t* zeroAt, bool scaled,
@@ -1962,7 +2045,7 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
     const oosg::DiagonalBlock* diagonalBlocks = p.dDiagonalBlocks.as<oosg::DiagonalBlock>();
     const oosg::AssemblyBlock* blocks = p.dBlocks.as<oosg::AssemblyBlock>();
     const oosg::AssemblyItem* items = p.dItems.as<oosg::AssemblyItem>();
-    const int2* inverseItems = p.dInverseItems.as<int2>();
+    const int4* inverseItems = p.dInverseItems.as<int4>();
     const oosg::UpdateTile* tiles = p.dTiles.as<oosg::UpdateTile>();
     const bool timing = p.timeLaunches;
     // The sweep ahead (a combined factorisation and solve): its levels are launched one at a time between the
@@ -2011,9 +2094,17 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
                   "factor: spool");
         check(hipEventRecord(p.oocFree[w], p.copyStream), "factor: spool");
     };
+    const bool concurrent = p.concurrent[sizeof(T) == sizeof(float) ? OOSG_FP32 : OOSG_FP64] && !p.profiler.enabled &&
+                            !p.outOfCore && !part;
+    // On one stream the whole inverses, which only the sweeps read, come after the last level, every level's together
+    // (a launch per height of the halvings and product, not per level); the sweep ahead and the level windows need
+    // theirs level by level, and the profile and the timing their own launches.
+    const bool merged = !concurrent && !p.profiler.enabled && !p.outOfCore && !part && !timing && p.aheadLevel <= 0;
     for (size_t li = 0; li < p.schedule.size(); ++li)
     {
         const Launch& l = p.schedule[li];
+        if (merged && l.kind == LaunchKind::Inverse)
+            continue;
         if (part && (l.kind == LaunchKind::Sync || l.level < levelFrom || l.level >= levelTo))
             continue;
         if (cancellable && li > 0 && l.level != p.schedule[li - 1].level)
@@ -2030,8 +2121,6 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
             panels = panelBase + (current % 2) * p.windowPanels;
             linv = linvBase + (current % 2) * p.windowLinv;
         }
-        const bool concurrent = p.concurrent[sizeof(T) == sizeof(float) ? OOSG_FP32 : OOSG_FP64] &&
-                                !p.profiler.enabled && !p.outOfCore && !part;
         if (p.aheadLevel > 0 && !aheadIssued && l.level >= p.aheadLevel)
         {
             // Everything launched so far is the factorisation of the levels below aheadLevel, on whichever streams
@@ -2112,6 +2201,8 @@ void runFactor(oosg_plan& p, const oosg_matrix& m, T* panels, T* linv, double* d
         if (timing)
             check(hipEventRecord(p.launchEvents[2 * li + 1], ls), "hipEventRecord");
     }
+    if (merged)
+        runMergedInverses<T>(p, panels, linv, st);
     while (aheadIssued && aheadNext < p.aheadLevel)
         aheadLevelLaunch();
     if (p.outOfCore && current >= 0)
@@ -2771,18 +2862,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
     check(oosg::launchUnitBlockInverses(d->dp, f.panels.as<double>(), f.linv.as<double>(),
                                         p.pivotInverseItems.as<int2>(), static_cast<int>(blockItems.size()), st),
           "factor: inverses");
-    for (int32_t l = 0; l < d->levels; ++l)
-        for (const oosg_plan::InverseRound& round : d->inverseRounds[l])
-        {
-            check(oosg::launchTriangleInverse<double>(d->dp, f.panels.as<double>(), f.linv.as<double>(),
-                                                      d->dInverseItems.as<int2>() + round.rowOffset, round.rowCount,
-                                                      -1, st),
-                  "factor: triangle inverses");
-            check(oosg::launchTriangleInverse<double>(d->dp, f.panels.as<double>(), f.linv.as<double>(),
-                                                      d->dInverseItems.as<int2>() + round.offset, round.count,
-                                                      round.step, st),
-                  "factor: triangle inverses");
-        }
+    runMergedInverses<double>(*d, f.panels.as<double>(), f.linv.as<double>(), st);
     f.dDiag = upload(pf->diag, st, "factor: pivots");
     pf->sub = upload(pf->sub_, st, "factor: pivots");
     pf->perm = upload(permOf, st, "factor: pivot order");

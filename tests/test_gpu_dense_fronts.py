@@ -1,9 +1,10 @@
 """Panels of dense fronts at the edges of the blocked elimination's blocks and tiles, on the GPU against numpy's Cholesky
 factor (L = C·diag(C)⁻¹, D = diag(C)²): a child of c columns over r rows and its parent of r columns, for c around the
-16-column sub-panels and the 64-column blocks of a panel step.
+16-column sub-panels and the 64-column blocks of a panel step, and where the triangle keeps its whole inverse (192
+columns and more: the solves read it).
 
 The matrices are symmetric with a dominating diagonal (condition below 4), so a backward-stable factor's entries differ
-from the exact ones by a few times n·eps of their type: below 1e-12 in FP64 and 1e-4 in FP32 for n <= 400."""
+from the exact ones by a few times n·eps of their type: below 1e-12 in FP64 and 1e-4 in FP32 for n <= 1200."""
 
 import numpy as np
 import pytest
@@ -27,7 +28,8 @@ def dense_front(c, r):
 
 @pytest.mark.parametrize("precision", [Precision.FP64, Precision.FP32])
 @pytest.mark.parametrize("c,r", [(1, 97), (15, 100), (16, 100), (17, 100), (33, 90), (48, 130), (63, 65), (64, 64),
-                                 (65, 64), (100, 1), (127, 33), (128, 128), (129, 100), (200, 150), (257, 130)])
+                                 (65, 64), (100, 1), (127, 33), (128, 128), (129, 100), (192, 40), (200, 150), (257, 130),
+                                 (449, 70), (1090, 60)])
 def test_panels_match_the_dense_factor(gpu_device, c, r, precision):
     dense, sym, matrix = dense_front(c, r)
     chol = np.linalg.cholesky(dense)
