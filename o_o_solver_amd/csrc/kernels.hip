@@ -2839,17 +2839,20 @@ __global__ __launch_bounds__(256) void columnMaxRowsKernel(const double* v, int6
 
 // ---- matrix values on the device ----------------------------------------------------------------------------------
 
+// Bound by HBM: 16 lanes to a column, its entries coalesced (a lane per column read each entry's line many times over:
+// 1.1 ms for the 41M entries of the 500 × 500 plate).
 __global__ __launch_bounds__(256) void combineValuesKernel(int32_t n, const int64_t* offsets, const int32_t* rows,
                                                            double alpha, const double* a, double beta,
                                                            const double* b, const double* scale, double* out,
                                                            double* diagonal, double* fp32Scale)
 {
 #pragma clang fp contract(off)
-    const int32_t j = int32_t(blockIdx.x) * 256 + int32_t(threadIdx.x);
+    const int32_t j = int32_t(blockIdx.x) * 16 + int32_t(threadIdx.x >> 4);
     if (j >= n)
         return;
     const int64_t k0 = offsets[j], k1 = offsets[j + 1];
-    for (int64_t k = k0; k < k1; ++k)
+    double d = 0.0;
+    for (int64_t k = k0 + (threadIdx.x & 15); k < k1; k += 16)
     {
         // Two products and a sum, each rounded (b null: the values of a as they are); then S·A·S as
         // scale[i]·a_ij·scale[j], left to right.
@@ -2866,8 +2869,11 @@ __global__ __launch_bounds__(256) void combineValuesKernel(int32_t n, const int6
             v = rowScaled * scale[j];
         }
         out[k] = v;
+        if (k == k0 && rows[k0] == j)
+            d = v;
     }
-    const double d = (k0 < k1 && rows[k0] == j) ? out[k0] : 0.0;
+    if ((threadIdx.x & 15) != 0)
+        return;
     diagonal[j] = d;
     double s = 1.0;
     if (d > 0.0 && isfinite(d))
@@ -2879,19 +2885,48 @@ __global__ __launch_bounds__(256) void combineValuesKernel(int32_t n, const int6
     fp32Scale[j] = s;
 }
 
+// Bound by HBM: a workgroup takes ROW_VALUES_ROWS consecutive rows, whose entries are one range of the CSR, by pieces of
+// ROW_VALUES_PIECE: read and written coalesced through LDS, from which a thread per row sums its entries in their order
+// (a thread per row from memory took 3.1 ms for the 80M entries of the 500 × 500 plate).
+constexpr int ROW_VALUES_ROWS = 128, ROW_VALUES_PIECE = 2048;
 __global__ __launch_bounds__(256) void rowValuesKernel(int32_t n, const int64_t* csrOffsets, const int64_t* map,
                                                        const double* values, double* csrValues,
                                                        unsigned long long* normKey)
 {
-    const int32_t i = int32_t(blockIdx.x) * 256 + int32_t(threadIdx.x);
+    __shared__ double piece[ROW_VALUES_PIECE];
+    const int32_t i0 = int32_t(blockIdx.x) * ROW_VALUES_ROWS, i1 = min(i0 + ROW_VALUES_ROWS, n);
+    const int32_t i = i0 + int32_t(threadIdx.x);
+    const bool owns = threadIdx.x < ROW_VALUES_ROWS && i < i1;
+    const int64_t from = csrOffsets[i0], to = csrOffsets[i1];
+    const int64_t e0 = owns ? csrOffsets[i] : 0, e1 = owns ? csrOffsets[i + 1] : 0;
     double sum = 0.0;
-    if (i < n)
-        for (int64_t e = csrOffsets[i]; e < csrOffsets[i + 1]; ++e)
+    for (int64_t base = from; base < to; base += ROW_VALUES_PIECE)
+    {
+        const int count = int(min(int64_t(ROW_VALUES_PIECE), to - base));
+        constexpr int PER = ROW_VALUES_PIECE / 256;
+        int64_t at[PER];
+        double v[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            at[q] = map[base + min(int(threadIdx.x) + 256 * q, count - 1)];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            v[q] = values[at[q]];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
         {
-            const double v = values[map[e]];
-            csrValues[e] = v;
-            sum += fabs(v);
+            const int e = int(threadIdx.x) + 256 * q;
+            if (e < count)
+            {
+                csrValues[base + e] = v[q];
+                piece[e] = fabs(v[q]);
+            }
         }
+        __syncthreads();
+        for (int64_t e = max(e0, base); e < min(e1, base + count); ++e)
+            sum += piece[e - base];
+        __syncthreads();
+    }
     // Non-negative doubles order as their bit patterns; a row whose sum is not a number is passed over, as the
     // host's std::max passes it over.
     const unsigned long long key = sum == sum ? __double_as_longlong(sum) : 0ull;
@@ -2901,7 +2936,7 @@ __global__ __launch_bounds__(256) void rowValuesKernel(int32_t n, const int64_t*
         const unsigned long long other = __shfl_xor(top, offset);
         top = other > top ? other : top;
     }
-    if ((threadIdx.x & 63) == 0)
+    if ((threadIdx.x & 63) == 0 && owns)
         atomicMax(normKey, top);
 }
 
@@ -3797,7 +3832,7 @@ hipError_t launchCombineValues(int32_t n, const int64_t* offsets, const int32_t*
                                double beta, const double* b, const double* scale, double* out, double* diagonal,
                                double* fp32Scale, hipStream_t stream)
 {
-    hipLaunchKernelGGL(combineValuesKernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, n,
+    hipLaunchKernelGGL(combineValuesKernel, dim3(static_cast<unsigned>((n + 15) / 16)), dim3(256), 0, stream, n,
                        offsets, rows, alpha, a, beta, b, scale, out, diagonal, fp32Scale);
     return hipGetLastError();
 }
@@ -3806,8 +3841,8 @@ hipError_t launchRowValues(int32_t n, const int64_t* csrOffsets, const int64_t* 
                            double* csrValues, unsigned long long* normKey, hipStream_t stream)
 {
     hipLaunchKernelGGL(fillInt32Kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<int32_t*>(normKey), 2, 0);
-    hipLaunchKernelGGL(rowValuesKernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, n,
-                       csrOffsets, map, values, csrValues, normKey);
+    hipLaunchKernelGGL(rowValuesKernel, dim3(static_cast<unsigned>((n + ROW_VALUES_ROWS - 1) / ROW_VALUES_ROWS)),
+                       dim3(256), 0, stream, n, csrOffsets, map, values, csrValues, normKey);
     return hipGetLastError();
 }
 

@@ -569,7 +569,9 @@ struct oosg_matrix
     int64_t nnz = 0;
     std::vector<int64_t> offsets;
     std::vector<int32_t> rows;
-    std::vector<double> diagonal; // a_jj, 0 when not stored
+    // a_jj, 0 when not stored (hostDiagonal: copied when first read after values set on the device).
+    mutable std::vector<double> diagonal;
+    mutable bool diagonalStale = false;
     std::vector<double> hostValues; // the values as last given
     std::vector<int64_t> csrFromCsc; // per CSR entry, its CSC entry
     double normInf = 0.0;
@@ -2253,6 +2255,16 @@ void releasePlan(oosg_plan* p)
     (void)hipGetLastError();
 }
 
+// The matrix diagonal on the host.
+const std::vector<double>& hostDiagonal(const oosg_matrix& m)
+{
+    if (m.diagonalStale && !m.diagonal.empty())
+        check(hipMemcpy(m.diagonal.data(), m.dDiagonal.ptr, m.diagonal.size() * sizeof(double), hipMemcpyDeviceToHost),
+              "matrix: diagonal");
+    m.diagonalStale = false;
+    return m.diagonal;
+}
+
 // The pivots of a positive definite factor on the host, copied on first use (FP32: d_j / s_j², those of the matrix).
 const std::vector<double>& hostDiagonal(const oosg_factor& f)
 {
@@ -2345,7 +2357,7 @@ void finish(const oosg_plan& p, const oosg_matrix& m, oosg_factor& f, const std:
     std::vector<int32_t> equations;
     for (int32_t j = 0; j < p.eliminated && f.issues.size() < OOSG_RECORDED_ISSUE_COUNT; ++j)
     {
-        const double diagonal = reference != nullptr && reference[j] >= 0.0 ? reference[j] : m.diagonal[j];
+        const double diagonal = reference != nullptr && reference[j] >= 0.0 ? reference[j] : hostDiagonal(m)[j];
         const double ratio = diagonal / d[j];
         const bool negative = ratio < 0.0 || d[j] < 0.0;
         if (ratio > maxRatio || negative)
@@ -4807,7 +4819,7 @@ oosg_status oosg_matrix_set_values(oosg_matrix* m, const double* values)
                   "matrix: row values");
             check(hipStreamSynchronize(st), "matrix: values");
             m->hostValues = std::move(v);
-            m->hostStale = false;
+            m->hostStale = m->diagonalStale = false;
         });
 }
 
@@ -4842,12 +4854,9 @@ void valuesChangedOnDevice(oosg_matrix& m)
           "matrix: rows");
     unsigned long long key = 0;
     check(hipMemcpyAsync(&key, m.dNormKey.ptr, sizeof(key), hipMemcpyDeviceToHost, st), "matrix: norm");
-    check(hipMemcpyAsync(m.diagonal.data(), m.dDiagonal.ptr, m.diagonal.size() * sizeof(double),
-                         hipMemcpyDeviceToHost, st),
-          "matrix: diagonal");
     check(hipStreamSynchronize(st), "matrix: values");
     std::memcpy(&m.normInf, &key, sizeof(double));
-    m.hostStale = true;
+    m.hostStale = m.diagonalStale = true;
 }
 
 } // namespace
