@@ -1900,32 +1900,41 @@ __global__ __launch_bounds__(64 * TINY_WAVES) void tinyBackwardKernel(DevicePlan
 // Wave-level: a 16-row tile (rows 16·tile within the block) of Inv·Y (TRANSPOSE: Invᵀ·Y) for the unit lower inverse of
 // the diagonal block of qb columns from row q0 (qb × qb column-major at inv), Y the block's rows of ys; the result in
 // the MFMA result layout.
-template <typename TP, bool TRANSPOSE>
-__device__ inline double4_t blockInverseTile(const TP* inv, int qb, int q0, const double* ys, int tile, int lr, int lq)
+template <typename TP> struct InverseTile
 {
-    const int i = 16 * tile + lr;
-    double a[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
+    TP a[16];
+    // The operands of tile `tile`'s rows, from positions clamped into the block (whose stored zeros are its other
+    // triangle's; rows beyond it give values that storeTile drops, columns beyond it meet zero rows of ys).
+    template <bool TRANSPOSE> __device__ inline void load(const TP* inv, int qb, int tile, int lr, int lq)
     {
-        const int j = 4 * q + lq;
-        const bool valid = i < qb && j < qb && (TRANSPOSE ? j >= i : j <= i);
-        const double value = double(inv[valid ? (TRANSPOSE ? j + i * qb : i + j * qb) : 0]);
-        a[q] = valid ? value : 0.0;
-    }
-    double4_t acc = {0.0, 0.0, 0.0, 0.0};
+        const int i = min(16 * tile + lr, qb - 1);
 #pragma unroll
-    for (int q = 0; q < 16; ++q)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], ys[(q0 + 4 * q + lq) * KMAX + lr], acc, 0, 0, 0);
-    return acc;
-}
+        for (int q = 0; q < 16; ++q)
+        {
+            const int j = min(4 * q + lq, qb - 1);
+            a[q] = inv[unsigned(TRANSPOSE ? j + i * qb : i + j * qb)];
+        }
+    }
+    __device__ inline double4_t times(const double* ys, int q0, int lr, int lq) const
+    {
+        double4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(double(pinned(a[q])), ys[(q0 + 4 * q + lq) * KMAX + lr], acc, 0,
+                                                       0, 0);
+        return acc;
+    }
+};
 
-// Stores a tile in the result layout to the rows row0 + lq + 4v of ys.
-__device__ inline void storeTile(double* ys, int row0, double4_t acc, int lr, int lq)
+// Stores a tile in the result layout to the rows row0 + lq + 4v of ys, zeros from row `end` on.
+__device__ inline void storeTile(double* ys, int row0, double4_t acc, int lr, int lq, int end)
 {
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-        ys[(row0 + lq + 4 * v) * KMAX + lr] = acc[v];
+    {
+        const int i = row0 + lq + 4 * v;
+        ys[i * KMAX + lr] = i < end ? acc[v] : 0.0;
+    }
 }
 
 __device__ inline double4_t loadTile(const double* ys, int row0, int lr, int lq)
@@ -1938,6 +1947,11 @@ __device__ inline double4_t loadTile(const double* ys, int row0, int lr, int lq)
 }
 
 // Forward: y_F = X(cols) (gathered), y_F ← L_FF⁻¹·y_F block by block, X(cols) = y_F, U(s) −= L_RF·y_F.
+//
+// Both kernels are bound by the latency of their chain of loads: so the triangle's operands are all loaded with the
+// supernode's own rows, the products below it take 32 values per lane at once (eight columns' or four tiles' loads in
+// flight before the first product), and every load goes unconditionally to a position clamped into its operand (a load
+// whose value feeds a select is waited for in a branch of its own).
 template <typename TP>
 __global__ __launch_bounds__(256) void mediumForwardKernel(DevicePlan p, const TP* panels, const TP* linv, double* X,
                                                            double* U, int k, const int32_t* list)
@@ -1945,126 +1959,141 @@ __global__ __launch_bounds__(256) void mediumForwardKernel(DevicePlan p, const T
     __shared__ double ys[MEDIUM_COLUMNS * KMAX];
     const int s = list[blockIdx.x];
     const int c = p.ncol[s], r = p.nrow[s], n = c + r, first = p.first[s];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
-    const int ct = (c + 15) >> 4;
-    for (int idx = tid; idx < MEDIUM_COLUMNS * KMAX; idx += 256)
-    {
-        const int i = idx >> 4, h = idx & (KMAX - 1);
-        const bool valid = i < c && h < k;
-        const double x = X[valid ? int64_t(first + i) * k + h : 0];
-        ys[idx] = valid ? x : 0.0;
-    }
-    __syncthreads();
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15,
+              lq = lane >> 4;
     const TP* L = panels + p.panelOff[s];
     const TP* inv = linv + p.linvOff[s];
-    const int qb0 = min(c, PANEL_BLOCK);
+    double* u = U + p.rowStart[s] * k;
+    double* x = X + int64_t(first) * k;
+    const int ct = (c + 15) >> 4, rt = (r + 15) >> 4;
+    const int qb0 = min(c, PANEL_BLOCK), qb1 = c - PANEL_BLOCK;
+    const int h = min(lr, k - 1); // columns from k on repeat the last, and are not stored
+    constexpr int PER = MEDIUM_COLUMNS * KMAX / 256;
+    double own[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        own[q] = x[unsigned(min((tid >> 4) + 16 * q, c - 1) * k + min(tid & (KMAX - 1), k - 1))];
+    InverseTile<TP> inverse0, inverse1;
+    TP l10[16];
+    if (16 * w < qb0)
+        inverse0.template load<false>(inv, qb0, w, lr, lq);
+    if (16 * w < qb1)
+    {
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            l10[q] = L[unsigned(PANEL_BLOCK + min(16 * w + lr, qb1 - 1) + (4 * q + lq) * n)];
+        inverse1.template load<false>(inv + PANEL_BLOCK * PANEL_BLOCK, qb1, w, lr, lq);
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        ys[tid + 256 * q] = (tid >> 4) + 16 * q < c ? pinned(own[q]) : 0.0;
+    __syncthreads();
     double4_t acc = {0.0, 0.0, 0.0, 0.0};
     if (16 * w < qb0)
-        acc = blockInverseTile<TP, false>(inv, qb0, 0, ys, w, lr, lq);
+        acc = inverse0.times(ys, 0, lr, lq);
     __syncthreads();
     if (16 * w < qb0)
-        storeTile(ys, 16 * w, acc, lr, lq);
+        storeTile(ys, 16 * w, acc, lr, lq, c);
     __syncthreads();
     if (c > PANEL_BLOCK)
     {
-        const int qb1 = c - PANEL_BLOCK;
         // y_1 −= L_10·z_0.
         if (16 * w < qb1)
         {
-            const int i = 16 * w + lr;
             acc = loadTile(ys, PANEL_BLOCK + 16 * w, lr, lq);
-            double a[16];
 #pragma unroll
             for (int q = 0; q < 16; ++q)
-            {
-                const int j = 4 * q + lq;
-                const bool valid = i < qb1;
-                const double value = double(L[valid ? (PANEL_BLOCK + i) + int64_t(j) * n : 0]);
-                a[q] = valid ? -value : 0.0;
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], ys[(4 * q + lq) * KMAX + lr], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-double(pinned(l10[q])), ys[(4 * q + lq) * KMAX + lr], acc,
+                                                           0, 0, 0);
         }
         __syncthreads();
         if (16 * w < qb1)
-            storeTile(ys, PANEL_BLOCK + 16 * w, acc, lr, lq);
+            storeTile(ys, PANEL_BLOCK + 16 * w, acc, lr, lq, c);
         __syncthreads();
         if (16 * w < qb1)
-            acc = blockInverseTile<TP, false>(inv + PANEL_BLOCK * PANEL_BLOCK, qb1, PANEL_BLOCK, ys, w, lr, lq);
+            acc = inverse1.times(ys, PANEL_BLOCK, lr, lq);
         __syncthreads();
         if (16 * w < qb1)
-            storeTile(ys, PANEL_BLOCK + 16 * w, acc, lr, lq);
+            storeTile(ys, PANEL_BLOCK + 16 * w, acc, lr, lq, c);
         __syncthreads();
     }
-    for (int idx = tid; idx < c * KMAX; idx += 256)
-    {
-        const int i = idx >> 4, h = idx & (KMAX - 1);
-        if (h < k)
-            X[int64_t(first + i) * k + h] = ys[idx];
-    }
-    // U(s) −= L_RF·y_F, 16-row tiles over the waves, the columns' k-steps 16 at a time.
-    double* u = U + p.rowStart[s] * k;
-    const int rt = (r + 15) >> 4, steps = 4 * ct;
+    if ((tid & (KMAX - 1)) < k)
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if ((tid >> 4) + 16 * q < c)
+                x[unsigned(((tid >> 4) + 16 * q) * k + (tid & (KMAX - 1)))] = ys[tid + 256 * q];
+    // U(s) −= L_RF·y_F, 16-row tiles over the waves; columns beyond c meet zero rows of ys.
     for (int t = w; t < rt; t += 4)
     {
-        const int rho = 16 * t + lr; // the A operand's row
+        const TP* row = L + (c + min(16 * t + lr, r - 1));
+        constexpr int STEPS = MEDIUM_COLUMNS / 4;
+        TP a[STEPS];
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-        {
-            const int i = 16 * t + lq + 4 * v;
-            const bool valid = i < r && lr < k;
-            const double value = u[valid ? int64_t(i) * k + lr : 0];
-            acc[v] = valid ? value : 0.0;
-        }
-        for (int q0 = 0; q0 < steps; q0 += 16)
-        {
-            double a[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
+        for (int g = 0; g < STEPS / 4; ++g)
+            if (g < ct)
             {
-                const int j = 4 * (q0 + q) + lq;
-                const bool valid = rho < r && j < c;
-                const double value = double(L[valid ? (c + rho) + int64_t(j) * n : 0]);
-                a[q] = valid ? -value : 0.0;
+#pragma unroll
+                for (int q = 4 * g; q < 4 * g + 4; ++q)
+                    a[q] = row[unsigned(min(4 * q + lq, c - 1) * n)];
             }
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
-                if (q0 + q < steps)
-                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], ys[(4 * (q0 + q) + lq) * KMAX + lr], acc, 0, 0,
-                                                               0);
-        }
+        for (int v = 0; v < 4; ++v)
+            acc[v] = u[unsigned(min(16 * t + lq + 4 * v, r - 1) * k + h)];
+#pragma unroll
+        for (int g = 0; g < STEPS / 4; ++g)
+            if (g < ct)
+            {
+                double y[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    y[q] = ys[(16 * g + 4 * q + lq) * KMAX + lr];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-double(pinned(a[4 * g + q])), y[q], acc, 0, 0, 0);
+            }
 #pragma unroll
         for (int v = 0; v < 4; ++v)
         {
             const int i = 16 * t + lq + 4 * v;
             if (i < r && lr < k)
-                u[int64_t(i) * k + lr] = acc[v];
+                u[unsigned(i * k + lr)] = acc[v];
         }
     }
 }
 
-// Backward: x_F = X(cols) − L_RFᵀ·X(rows) (wave w: the columns' tiles w and w + 4 over every row below), then
+// Backward: x_F = X(cols) − L_RFᵀ·X(rows) (the waves take batches of 32 rows over every column tile), then
 // X(cols) = L_FF⁻ᵀ·x_F block by block from the last.
 template <typename TP>
-__global__ __launch_bounds__(256) void mediumBackwardKernel(DevicePlan p, const TP* panels, const TP* linv, double* X,
+__global__ __launch_bounds__(256, 2) void mediumBackwardKernel(DevicePlan p, const TP* panels, const TP* linv, double* X,
                                                             int k, const int32_t* list)
 {
     __shared__ double xs[MEDIUM_COLUMNS * KMAX];
     const int s = list[blockIdx.x];
     const int c = p.ncol[s], r = p.nrow[s], n = c + r, first = p.first[s];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15,
+              lq = lane >> 4;
     const int ct = (c + 15) >> 4;
+    const int qb0 = min(c, PANEL_BLOCK), qb1 = c - PANEL_BLOCK;
+    const int h = min(lr, k - 1); // columns from k on repeat the last, and are not stored
     const TP* L = panels + p.panelOff[s];
+    const TP* inv = linv + p.linvOff[s];
     const int32_t* rows = p.rows + p.rowStart[s];
+    double* x = X + int64_t(first) * k;
+    constexpr int TILES = MEDIUM_COLUMNS / 16;
+    // The supernode's own rows and the triangle's operands, used after the products below it.
+    double4_t own[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            own[e][v] = x[unsigned(min(16 * (w + 4 * e) + lq + 4 * v, c - 1) * k + h)];
     // The first MEDIUM_ROW_INDICES row indices through LDS (one coalesced load), the rest read where used.
     __shared__ int32_t rowIndex[MEDIUM_ROW_INDICES];
     for (int i = tid; i < min(r, MEDIUM_ROW_INDICES); i += 256)
         rowIndex[i] = rows[i];
     __syncthreads();
-    // x_F −= L_RFᵀ·X(rows): wave w takes the batches of 32 rows w, w + 4, ... over every column tile, its partial sums
-    // in registers; each batch's X rows (rows r0 + 4m + lq) are gathered while the previous batch is multiplied.
-    constexpr int TILES = MEDIUM_COLUMNS / 16;
+    // x_F −= L_RFᵀ·X(rows): wave w takes the batches of 32 rows w, w + 4, ..., its partial sums in registers; each
+    // batch's X rows (rows r0 + 4m + lq) are gathered while the previous batch is multiplied.
     double4_t part[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
@@ -2074,118 +2103,111 @@ __global__ __launch_bounds__(256) void mediumBackwardKernel(DevicePlan p, const 
 #pragma unroll
         for (int m = 0; m < 8; ++m)
         {
-            const int rho = r0 + 4 * m + lq;
-            const bool valid = rho < r && lr < k;
-            const int32_t row = rho < MEDIUM_ROW_INDICES ? rowIndex[rho < r ? rho : 0] : rows[rho < r ? rho : 0];
-            const double value = X[valid ? int64_t(row) * k + lr : 0];
-            b[m] = valid ? value : 0.0;
+            const int rho = min(r0 + 4 * m + lq, r - 1);
+            const int32_t row = rho < MEDIUM_ROW_INDICES ? rowIndex[rho] : rows[rho];
+            b[m] = X[int64_t(row) * k + h];
         }
     };
     double next[8];
-    gatherBatch(32 * w, next);
+    if (32 * w < r)
+        gatherBatch(32 * w, next);
     for (int r0 = 32 * w; r0 < r; r0 += 128)
     {
         double b[8];
 #pragma unroll
         for (int m = 0; m < 8; ++m)
-            b[m] = next[m];
+            b[m] = r0 + 4 * m + lq < r ? pinned(next[m]) : 0.0; // rows beyond the last: zero
         if (r0 + 128 < r)
             gatherBatch(r0 + 128, next);
+        // Four column tiles at a time: lane row j of tile t is column j of L.
 #pragma unroll
-        for (int t = 0; t < TILES; ++t)
-            if (t < ct)
+        for (int t0 = 0; t0 < TILES; t0 += 4)
+            if (t0 < ct)
             {
-                const int j = 16 * t + lr; // the A operand's row: column j of L
-                double a[8];
+                TP a[4][8];
 #pragma unroll
-                for (int m = 0; m < 8; ++m)
-                {
-                    const int rho = r0 + 4 * m + lq;
-                    const bool valid = rho < r && j < c;
-                    const double value = double(L[valid ? (c + rho) + int64_t(j) * n : 0]);
-                    a[m] = valid ? -value : 0.0;
-                }
+                for (int t = 0; t < 4; ++t)
+                    if (t0 + t < ct)
+                    {
+                        const TP* column = L + c + int64_t(min(16 * (t0 + t) + lr, c - 1)) * n;
 #pragma unroll
-                for (int m = 0; m < 8; ++m)
-                    part[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], b[m], part[t], 0, 0, 0);
+                        for (int m = 0; m < 8; ++m)
+                            a[t][m] = column[min(r0 + 4 * m + lq, r - 1)];
+                    }
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (t0 + t < ct)
+                    {
+#pragma unroll
+                        for (int m = 0; m < 8; ++m)
+                            part[t0 + t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-double(pinned(a[t][m])), b[m],
+                                                                                part[t0 + t], 0, 0, 0);
+                    }
             }
     }
-    // x_F = X(cols) + the waves' sums, added in wave order through LDS (every tile written by wave 0: zeros beyond
-    // the columns).
+    InverseTile<TP> inverse0, inverse1;
+    TP l10[16];
+    if (16 * w < qb0)
+        inverse0.template load<true>(inv, qb0, w, lr, lq);
+    if (c > PANEL_BLOCK)
+    {
+        if (16 * w < qb1)
+            inverse1.template load<true>(inv + PANEL_BLOCK * PANEL_BLOCK, qb1, w, lr, lq);
+        // L_10ᵀ: row i is column i of L; its columns beyond qb1 meet zero rows of xs.
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            l10[q] = L[unsigned(PANEL_BLOCK + min(4 * q + lq, qb1 - 1) + (16 * w + lr) * n)];
+    }
+    // x_F = X(cols) + the waves' sums, added in wave order through LDS: first X(cols) (zeros beyond the columns).
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        storeTile(xs, 16 * (w + 4 * e), own[e], lr, lq, c);
+    __syncthreads();
     for (int q = 0; q < 4; ++q)
     {
         if (w == q)
 #pragma unroll
             for (int t = 0; t < TILES; ++t)
-            {
-                double4_t base;
-                if (q == 0)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                    {
-                        const int i = 16 * t + lq + 4 * v;
-                        const bool valid = i < c && lr < k;
-                        const double value = X[valid ? int64_t(first + i) * k + lr : 0];
-                        base[v] = valid ? value : 0.0;
-                    }
-                else if (t < ct)
-                    base = loadTile(xs, 16 * t, lr, lq);
-                if (q == 0 || t < ct)
+                if (t < ct)
                 {
+                    double4_t base = loadTile(xs, 16 * t, lr, lq);
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
                         base[v] += part[t][v];
-                    storeTile(xs, 16 * t, base, lr, lq);
+                    storeTile(xs, 16 * t, base, lr, lq, c);
                 }
-            }
         __syncthreads();
     }
-    const TP* inv = linv + p.linvOff[s];
-    const int qb0 = min(c, PANEL_BLOCK);
     double4_t t0 = {0.0, 0.0, 0.0, 0.0};
     if (c > PANEL_BLOCK)
     {
-        const int qb1 = c - PANEL_BLOCK;
         if (16 * w < qb1)
-            t0 = blockInverseTile<TP, true>(inv + PANEL_BLOCK * PANEL_BLOCK, qb1, PANEL_BLOCK, xs, w, lr, lq);
+            t0 = inverse1.times(xs, PANEL_BLOCK, lr, lq);
         __syncthreads();
         if (16 * w < qb1)
-            storeTile(xs, PANEL_BLOCK + 16 * w, t0, lr, lq);
+            storeTile(xs, PANEL_BLOCK + 16 * w, t0, lr, lq, c);
         __syncthreads();
         // x_0 −= L_10ᵀ·z_1.
-        {
-            const int i = 16 * w + lr; // row i of L_10ᵀ: column i of L
-            t0 = loadTile(xs, 16 * w, lr, lq);
-            double a[16];
+        t0 = loadTile(xs, 16 * w, lr, lq);
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
-            {
-                const int j = 4 * q + lq; // row PANEL_BLOCK + j of L
-                const bool valid = j < qb1;
-                const double value = double(L[valid ? (PANEL_BLOCK + j) + int64_t(i) * n : 0]);
-                a[q] = valid ? -value : 0.0;
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-                t0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], xs[(PANEL_BLOCK + 4 * q + lq) * KMAX + lr], t0, 0, 0,
-                                                          0);
-        }
+        for (int q = 0; q < 16; ++q)
+            t0 = __builtin_amdgcn_mfma_f64_16x16x4f64(-double(pinned(l10[q])),
+                                                      xs[(PANEL_BLOCK + 4 * q + lq) * KMAX + lr], t0, 0, 0, 0);
         __syncthreads();
-        storeTile(xs, 16 * w, t0, lr, lq);
+        storeTile(xs, 16 * w, t0, lr, lq, c);
         __syncthreads();
     }
     if (16 * w < qb0)
-        t0 = blockInverseTile<TP, true>(inv, qb0, 0, xs, w, lr, lq);
+        t0 = inverse0.times(xs, 0, lr, lq);
     __syncthreads();
     if (16 * w < qb0)
-        storeTile(xs, 16 * w, t0, lr, lq);
+        storeTile(xs, 16 * w, t0, lr, lq, c);
     __syncthreads();
-    for (int idx = tid; idx < c * KMAX; idx += 256)
-    {
-        const int i = idx >> 4, h = idx & (KMAX - 1);
-        if (h < k)
-            X[int64_t(first + i) * k + h] = xs[idx];
-    }
+    if ((tid & (KMAX - 1)) < k)
+#pragma unroll
+        for (int q = 0; q < MEDIUM_COLUMNS * KMAX / 256; ++q)
+            if ((tid >> 4) + 16 * q < c)
+                x[unsigned(((tid >> 4) + 16 * q) * k + (tid & (KMAX - 1)))] = xs[tid + 256 * q];
 }
 
 // The update vectors of the big supernodes of a level: U(s)(rows of the tile) −= L_RF(tile, :)·X(cols(s)).
