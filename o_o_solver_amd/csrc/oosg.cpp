@@ -2460,6 +2460,156 @@ void addPivotTiles(std::vector<oosg::UpdateTile>& tiles, int64_t fOff, int64_t w
         }
 }
 
+// The rows and relative indices of a pivoted factor's structure d (its columns, row counts and tree set): rows in pivot
+// order, each child's rows at their positions among its parent's panel rows.
+void pivotedStructure(const oosg_plan& p, oosg_plan& d, const PivotedFactor& pf,
+                      const std::vector<std::vector<int32_t>>& frontRows)
+{
+    const int32_t S = p.S, n = p.n;
+    d.rowStart.assign(S + 1, 0);
+    for (int32_t s = 0; s < S; ++s)
+        d.rowStart[s + 1] = d.rowStart[s] + d.nrow[s];
+    d.rows.resize(static_cast<size_t>(d.rowStart[S]));
+    d.rel.assign(d.rows.size(), 0);
+    for (int32_t s = 0; s < S; ++s)
+        for (int32_t i = 0; i < d.nrow[s]; ++i)
+            d.rows[d.rowStart[s] + i] = pf.pivotOf[frontRows[s][pf.eliminated[s] + i]];
+    {
+        // Each child's rows → positions in its parent's panel rows.
+        std::vector<int32_t> posOf(static_cast<size_t>(n), -1);
+        for (int32_t s = 0; s < S; ++s)
+        {
+            if (p.childStart[s] == p.childStart[s + 1])
+                continue;
+            for (int32_t k = 0; k < pf.order[s]; ++k)
+                posOf[frontRows[s][k]] = k;
+            for (int32_t x = p.childStart[s]; x < p.childStart[s + 1]; ++x)
+            {
+                const int32_t ch = p.children[x];
+                for (int32_t i = 0; i < d.nrow[ch]; ++i)
+                {
+                    const int32_t at = posOf[frontRows[ch][pf.eliminated[ch] + i]];
+                    if (at < 0)
+                        fail(OOSG_INTERNAL, "factor: a row of a child is not in its parent's front");
+                    d.rel[d.rowStart[ch] + i] = at;
+                }
+            }
+            for (int32_t k = 0; k < pf.order[s]; ++k)
+                posOf[frontRows[s][k]] = -1;
+        }
+    }
+    for (int32_t s = 0; s < S; ++s)
+        if (d.parent[s] < 0 && d.nrow[s] > 0)
+            fail(OOSG_INTERNAL, "factor: a root front kept rows");
+}
+
+// The same structure and its sweep plan where no column was delayed: the plan's own, every supernode with its columns
+// and rows where they were but its candidates interchanged among themselves. Its lists are the plan's (their device
+// arrays are shared: the factor holds the plan); only the rows' equations, and the positions of the supernodes that
+// interchanged, change. Deriving and uploading them anew was host work with the GPU idle: a shifted factorisation and
+// two solves of the 360 × 200 cylinder took 91 ms with it and take 78 ms without, of the 48 × 20 one 5.2 and 4.8 ms.
+// A delayed column changes the sizes of two fronts and with them every offset and list: those factors derive anew.
+void permuteSweepPlan(const oosg_plan& p, oosg_plan& d, const PivotedFactor& pf,
+                      const std::vector<std::vector<int32_t>>& frontRows)
+{
+    const hipStream_t st = d.stream;
+    d.rowStart = p.rowStart;
+    d.panelOff = p.panelOff;
+    d.updateOff = p.updateOff;
+    d.linvOff = p.linvOff;
+    d.levels = p.levels;
+    d.levelStart = p.levelStart;
+    d.levelList = p.levelList;
+    d.levelOf = p.levelOf;
+    d.levelPanelValues = p.levelPanelValues;
+    d.sweepWork = p.sweepWork;
+    d.flops = p.flops;
+    d.partialSlots = p.partialSlots;
+    d.tinyStart = p.tinyStart;
+    d.otherStart = p.otherStart;
+    d.mediumStart = p.mediumStart;
+    d.pullWidth = p.pullWidth;
+    d.gatherChunkStart = p.gatherChunkStart;
+    d.forwardTileStart = p.forwardTileStart;
+    d.backwardBlockStart = p.backwardBlockStart;
+    d.forwardSubtractionStart = p.forwardSubtractionStart;
+    d.backwardSubtractionStart = p.backwardSubtractionStart;
+    d.forwardTriangleStart = p.forwardTriangleStart;
+    d.backwardTriangleStart = p.backwardTriangleStart;
+    d.triangleSumStart = p.triangleSumStart;
+    d.mergedInverses = p.mergedInverses;
+    d.rows.resize(p.rows.size());
+    for (size_t e = 0; e < p.rows.size(); ++e)
+        d.rows[e] = pf.pivotOf[p.rows[e]];
+    d.rel = p.rel;
+    std::vector<int32_t> pulls, gatherStart, gatherRows;
+    std::vector<int32_t> to; // a candidate's position after the interchanges
+    for (int32_t s = 0; s < p.S; ++s)
+    {
+        const int32_t c = p.ncol[s];
+        bool moved = false;
+        for (int32_t k = 0; k < c && !moved; ++k)
+            moved = frontRows[s][k] != p.first[s] + k;
+        if (!moved)
+            continue;
+        to.assign(static_cast<size_t>(c), 0);
+        for (int32_t k = 0; k < c; ++k)
+            to[frontRows[s][k] - p.first[s]] = k;
+        for (int32_t x = p.childStart[s]; x < p.childStart[s + 1]; ++x)
+            for (int64_t e = p.rowStart[p.children[x]]; e < p.rowStart[p.children[x] + 1]; ++e)
+                if (p.rel[e] < c)
+                    d.rel[e] = to[p.rel[e]];
+        if (gatherStart.empty())
+        {
+            pulls = p.pulls;
+            gatherStart = p.gatherStart;
+            gatherRows = p.gatherRows;
+        }
+        if (p.pullBase[s] >= 0)
+            for (int32_t q = 0; q < c; ++q)
+                for (int t = 0; t < oosg::TINY_PULLS; ++t)
+                    pulls[(static_cast<size_t>(p.pullBase[s]) + to[q]) * oosg::TINY_PULLS + t] =
+                        p.pulls[(static_cast<size_t>(p.pullBase[s]) + q) * oosg::TINY_PULLS + t];
+        if (p.otherPosStart[s] >= 0)
+        {
+            const size_t base = static_cast<size_t>(p.otherPosStart[s]);
+            int32_t at = p.gatherStart[base];
+            for (int32_t k = 0; k < c; ++k)
+            {
+                const size_t from = base + static_cast<size_t>(frontRows[s][k] - p.first[s]);
+                gatherStart[base + k] = at;
+                for (int32_t e = p.gatherStart[from]; e < p.gatherStart[from + 1]; ++e)
+                    gatherRows[at++] = p.gatherRows[e];
+            }
+        }
+    }
+    const auto share = [](const DeviceBuffer& b) { return DeviceBuffer::view(b.ptr, b.bytes); };
+    d.dTinyList = share(p.dTinyList);
+    d.dOtherList = share(p.dOtherList);
+    d.dMediumList = share(p.dMediumList);
+    d.dGatherChunks = share(p.dGatherChunks);
+    d.dForwardTiles = share(p.dForwardTiles);
+    d.dBackwardBlocks = share(p.dBackwardBlocks);
+    d.dForwardSubtractions = share(p.dForwardSubtractions);
+    d.dBackwardSubtractions = share(p.dBackwardSubtractions);
+    d.dForwardTriangles = share(p.dForwardTriangles);
+    d.dBackwardTriangles = share(p.dBackwardTriangles);
+    d.dForwardTriangleSums = share(p.dForwardTriangleSums);
+    d.dBackwardTriangleSums = share(p.dBackwardTriangleSums);
+    d.dInverseItems = share(p.dInverseItems);
+    d.dRows = upload(d.rows, st, "factor: rows");
+    d.dRel = upload(d.rel, st, "factor: relative indices");
+    const bool interchanged = !gatherStart.empty();
+    d.dPulls = interchanged ? upload(pulls, st, "factor: pull table") : share(p.dPulls);
+    d.dGatherStart = interchanged ? upload(gatherStart, st, "factor: gather lists") : share(p.dGatherStart);
+    d.dGatherRows = interchanged ? upload(gatherRows, st, "factor: gather lists") : share(p.dGatherRows);
+    d.dp = p.dp;
+    d.dp.rows = d.dRows.as<int32_t>();
+    d.dp.rel = d.dRel.as<int32_t>();
+    d.dp.pulls = d.dPulls.as<int4>();
+    check(hipStreamSynchronize(st), "factor: sweep plan");
+}
+
 // The indefinite factorisation (MultifrontalDriver::eliminatePivoted, MultifrontalDriver.cpp:346-436), level by level:
 // each front [own columns, the columns its children delayed (in child order), rows] is assembled, eliminated with
 // Bunch–Kaufman pivoting among its candidates in blocks of PANEL_BLOCK columns, the candidates it cannot eliminate
@@ -2819,43 +2969,14 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
     pf->panelRows.reserve(static_cast<size_t>(pf->rowsStart[S]));
     for (int32_t s = 0; s < S; ++s)
         pf->panelRows.insert(pf->panelRows.end(), frontRows[s].begin(), frontRows[s].end());
-    d->rowStart.assign(S + 1, 0);
-    for (int32_t s = 0; s < S; ++s)
-        d->rowStart[s + 1] = d->rowStart[s] + d->nrow[s];
-    d->rows.resize(static_cast<size_t>(d->rowStart[S]));
-    d->rel.assign(d->rows.size(), 0);
-    for (int32_t s = 0; s < S; ++s)
-        for (int32_t i = 0; i < d->nrow[s]; ++i)
-            d->rows[d->rowStart[s] + i] = pf->pivotOf[frontRows[s][pf->eliminated[s] + i]];
+    if (pf->delayed == 0 && p.trailing < 0 && !p.outOfCore && d->first == p.first)
+        permuteSweepPlan(p, *d, *pf, frontRows);
+    else
     {
-        // Each child's rows → positions in its parent's panel rows.
-        std::vector<int32_t> posOf(static_cast<size_t>(n), -1);
-        for (int32_t s = 0; s < S; ++s)
-        {
-            if (p.childStart[s] == p.childStart[s + 1])
-                continue;
-            for (int32_t k = 0; k < pf->order[s]; ++k)
-                posOf[frontRows[s][k]] = k;
-            for (int32_t x = p.childStart[s]; x < p.childStart[s + 1]; ++x)
-            {
-                const int32_t ch = p.children[x];
-                for (int32_t i = 0; i < d->nrow[ch]; ++i)
-                {
-                    const int32_t at = posOf[frontRows[ch][pf->eliminated[ch] + i]];
-                    if (at < 0)
-                        fail(OOSG_INTERNAL, "factor: a row of a child is not in its parent's front");
-                    d->rel[d->rowStart[ch] + i] = at;
-                }
-            }
-            for (int32_t k = 0; k < pf->order[s]; ++k)
-                posOf[frontRows[s][k]] = -1;
-        }
+        pivotedStructure(p, *d, *pf, frontRows);
+        deriveLevels(*d);
+        uploadSweepPlan(*d);
     }
-    for (int32_t s = 0; s < S; ++s)
-        if (d->parent[s] < 0 && d->nrow[s] > 0)
-            fail(OOSG_INTERNAL, "factor: a root front kept rows");
-    deriveLevels(*d);
-    uploadSweepPlan(*d);
     // The inverses of the unit lower triangles: the diagonal blocks, then the wide triangles' whole inverses.
     allocateCounted(p, f.linv, static_cast<size_t>(std::max<int64_t>(d->linvOff[S], 1)) * sizeof(double),
                     "factor: inverses");

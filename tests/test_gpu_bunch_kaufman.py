@@ -259,3 +259,45 @@ def test_delayed_columns_keep_the_inertia(gpu_device, sizes, seed):
     b = rng.standard_normal((n, 2))
     x = FactorSolve(f).solve(b)
     assert backward_error(m, x, b) <= 1e-12
+
+
+@pytest.mark.parametrize("nx,k", [(8, 1), (30, 5), (60, 17)])
+def test_interchanges_without_delays_solve_as_the_general_structure_does(gpu_device, nx, k):
+    # A plate whose supernodes interchange among their own columns but delay none (couplings to the rows below 1e-3 of
+    # those within), with seven equations of their own appended: with a strong block there no column of the factor is
+    # delayed, and the sweeps' lists are the plan's; with a weak one its columns are, and the lists are derived anew.
+    # The plate's equations see the same operations either way: the same panels, and solutions equal to the last bit.
+    w = models.plate(nx)
+    sym = w.analyse()
+    p = w.matrix
+    n, s = p.n, sym.supernode_count
+    union = SymbolicFactor(n + 7, np.concatenate([sym.first_column, [n, n + 4]]),
+                           np.concatenate([sym.column_count, [4, 3]]), np.concatenate([sym.parent, [s + 1, -1]]),
+                           np.concatenate([sym.row_start, np.array([3, 3]) + sym.row_start[-1]]),
+                           np.concatenate([sym.rows_all, [n + 4, n + 5, n + 6]]).astype(np.int32))
+    rng = np.random.default_rng(nx)
+    own = np.repeat(np.arange(s), sym.column_count)
+    cols = np.repeat(np.arange(n), np.diff(p.offsets))
+    values = rng.standard_normal(len(p.rows)) * np.where(own[p.rows] == own[cols], 1.0, 1e-3)
+    block = np.tril(rng.standard_normal((7, 7)))
+    b = rng.standard_normal((n + 7, k))
+    solved = []
+    for weak in (False, True):
+        dense = block.copy()
+        dense[:4, :4] *= 1e-6 if weak else 1e3
+        m = SymmetricCsc(n + 7, np.concatenate([p.offsets, p.offsets[-1] + np.cumsum(np.arange(7, 0, -1))]),
+                         np.concatenate([p.rows] + [np.arange(n + j, n + 7) for j in range(7)]).astype(np.int32),
+                         np.concatenate([values] + [dense[j:, j] for j in range(7)]))
+        f = SupernodalFactor.factorise(union, m, INDEFINITE)
+        assert (f.delayed_pivot_count > 0) == weak
+        x = FactorSolve(f).solve(b)
+        assert backward_error(m, x, b) <= 1e-12
+        solved.append((f, x))
+    strong, general = solved[0][0], solved[1][0]
+    moved = 0
+    for q in range(s):
+        (panel, rows), (other, other_rows) = strong.panel(q), general.panel(q)
+        assert rows.tolist() == other_rows.tolist() and np.array_equal(panel, other)
+        moved += rows.tolist() != sorted(rows.tolist())
+    assert moved > s // 4
+    assert np.array_equal(solved[0][1][:n], solved[1][1][:n])
