@@ -223,13 +223,13 @@ hipError_t launchExtendTiles(const DevicePlan& p, T* panels, T* updates, const U
 template <typename T>
 hipError_t launchUpdateTiles(const DevicePlan& p, T* panels, T* updates, T* linv, const UpdateTile* tiles, int count,
                              double* diagOut, int32_t* zeroAt, bool fused, hipStream_t stream);
-// One level of the forward sweep: the supernodes of `list`, then the row tiles (supernode, tile) of its big ones.
+// One level of the forward sweep: the supernodes of `list` (gathered, below WIDE_COLUMNS columns), then the row tiles (supernode, tile) of its big ones.
 template <typename TP>
 hipError_t launchForward(const DevicePlan& p, const TP* panels, const TP* linv, double* X, double* U, int k,
                          const int32_t* list, int count, const int4* rowTiles, int tileCount, double* partials,
-                         hipStream_t stream, bool gathered = false);
+                         hipStream_t stream);
 // The gathers of a level's other supernodes, by chunks of GATHER_CHUNK front positions: X(cols) += and U(rows) = the
-// children's update rows, before launchForward(gathered). A chunk: its first position q0 in the front of its supernode
+// children's update rows, before launchForward. A chunk: its first position q0 in the front of its supernode
 // (order c + r, c columns from `first`, update rows from `rowStart`), the front's first position in the gather lists.
 constexpr int GATHER_CHUNK = 16;
 struct GatherChunk

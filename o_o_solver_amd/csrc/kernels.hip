@@ -1424,12 +1424,6 @@ __device__ inline int accColumn()
     return threadIdx.x & 15;
 }
 
-// Wide supernodes solve their triangles by the whole inverse (triangleProductsKernel).
-__device__ inline bool isWideSupernode(int c)
-{
-    return keepsTriangleInverse(c);
-}
-
 // ys ← inv·ys (transpose: invᵀ·ys) for the unit lower inverse of a diagonal block (column-major qb × qb), staged in
 // blk and applied by MFMA; ys is SB × KMAX, zero beyond its rows and columns.
 template <typename TP>
@@ -1517,63 +1511,14 @@ __device__ inline void storeBlockRows(const double* ys, double* X, int64_t row0,
 
 template <typename TP>
 __global__ __launch_bounds__(256) void forwardKernel(DevicePlan p, const TP* panels, const TP* linv, double* X,
-                                                     double* U, int k, const int32_t* list, int gathered)
+                                                     double* U, int k, const int32_t* list)
 {
     __shared__ TP blk[SB * SBP];
     __shared__ double ys[SB * KMAX];
     const int s = list[blockIdx.x];
     const int c = p.ncol[s], r = p.nrow[s], n = c + r, first = p.first[s];
-    if (gathered && isWideSupernode(c))
-        return; // its gather is done (gatherKernel), its triangle is a product with the whole inverse
     const TP* L = panels + p.panelOff[s];
     double* u = U + p.rowStart[s] * k;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    if (!gathered)
-        for (int idx = tid; idx < r * k; idx += nt)
-            u[idx] = 0.0;
-    for (int q = p.childStart[s]; q < p.childStart[s + 1] && !gathered; ++q)
-    {
-        __syncthreads();
-        const int ch = p.children[q];
-        const int rc = p.nrow[ch];
-        const int32_t* rel = p.rel + p.rowStart[ch];
-        const double* uc = U + p.rowStart[ch] * k;
-        // Eight elements (i, h) of the child's rc × k values per thread per pass (distinct targets: a child's rows
-        // map to distinct rows of s): the child's values and positions are loaded first (from elements clamped into
-        // its values), then the eight targets, then the eight sums are stored.
-        constexpr int UNROLL = 8;
-        const int total = rc * k;
-        for (int base = tid; base < total; base += UNROLL * nt)
-        {
-            int pos[UNROLL], col[UNROLL];
-            double v[UNROLL];
-#pragma unroll
-            for (int t = 0; t < UNROLL; ++t)
-            {
-                const int idx = min(base + t * nt, total - 1);
-                const int i = idx / k;
-                col[t] = idx - i * k;
-                pos[t] = rel[i];
-                v[t] = uc[idx];
-            }
-            double* y[UNROLL];
-            double old[UNROLL];
-#pragma unroll
-            for (int t = 0; t < UNROLL; ++t)
-            {
-                const int at = pinned(pos[t]);
-                y[t] = at < c ? X + int64_t(first + at) * k + col[t] : u + int64_t(at - c) * k + col[t];
-                old[t] = *y[t];
-            }
-#pragma unroll
-            for (int t = 0; t < UNROLL; ++t)
-                if (base + t * nt < total)
-                    *y[t] = pinned(old[t]) + pinned(v[t]);
-        }
-    }
-    __syncthreads();
-    if (isWideSupernode(c))
-        return; // its triangle is a product with the whole inverse (triangleProductsKernel)
     // The triangle L_FF, and the rows below (L_RF) of a small supernode; a larger one's are the row tiles of
     // forwardRowsKernel.
     const int rowsEnd = sweepRowsInline(c, r) ? n : c;
@@ -2391,8 +2336,8 @@ __global__ __launch_bounds__(256) void backwardKernel(DevicePlan p, const TP* pa
     __shared__ double ys[SB * KMAX];
     const int s = list[blockIdx.x];
     const int c = p.ncol[s], r = p.nrow[s], n = c + r, first = p.first[s];
-    if (isWideSupernode(c) || c == 0)
-        return; // backwardColumnsKernel and triangleProductsKernel did it; or no columns (all delayed)
+    if (c == 0)
+        return; // no columns (all delayed)
     const TP* L = panels + p.panelOff[s];
     const int32_t* rows = p.rows + p.rowStart[s];
     const int h = accColumn();
@@ -3382,11 +3327,10 @@ hipError_t launchMediumBackward(const DevicePlan& p, const TP* panels, const TP*
 template <typename TP>
 hipError_t launchForward(const DevicePlan& p, const TP* panels, const TP* linv, double* X, double* U, int k,
                          const int32_t* list, int count, const int4* rowTiles, int tileCount, double* partials,
-                         hipStream_t stream, bool gathered)
+                         hipStream_t stream)
 {
     if (count > 0)
-        hipLaunchKernelGGL(forwardKernel<TP>, dim3(count), dim3(256), 0, stream, p, panels, linv, X, U, k, list,
-                           gathered ? 1 : 0);
+        hipLaunchKernelGGL(forwardKernel<TP>, dim3(count), dim3(256), 0, stream, p, panels, linv, X, U, k, list);
     if (tileCount > 0)
         hipLaunchKernelGGL(forwardRowsKernel<TP>, dim3(tileCount), dim3(256), 0, stream, p, panels, X, U, k,
                            rowTiles, partials);
@@ -4099,7 +4043,7 @@ hipError_t launchMfmaProbe(const double* a, const double* b, double* d, const fl
     template hipError_t launchExtendTiles<T>(const DevicePlan&, T*, T*, const UpdateTile*, int, const int32_t*,        \
                                              const AssemblyItem*, int, hipStream_t);                                   \
     template hipError_t launchForward<T>(const DevicePlan&, const T*, const T*, double*, double*, int, const int32_t*, \
-                                         int, const int4*, int, double*, hipStream_t, bool);                           \
+                                         int, const int4*, int, double*, hipStream_t);                                 \
     template hipError_t launchBackward<T>(const DevicePlan&, const T*, const T*, double*, int, const int32_t*, int,     \
                                           const int4*, int, double*, hipStream_t);                                     \
     template hipError_t launchMediumForward<T>(const DevicePlan&, const T*, const T*, double*, double*, int,           \
