@@ -1839,12 +1839,12 @@ __global__ __launch_bounds__(64 * TINY_WAVES) void tinyBackwardKernel(DevicePlan
 // Supernodes of at most MEDIUM_COLUMNS columns that are not tiny are swept by one workgroup of four waves each, with
 // FP64 MFMA products: the right-hand sides of the front's columns in LDS (MEDIUM_COLUMNS × KMAX doubles, zero beyond
 // its rows and columns), the triangle by the inverses of its diagonal blocks of PANEL_BLOCK columns (two at most), a
-// wave per 16-row tile of a block; the rows below in 16-row tiles spread over the waves (forward), the columns' tiles
-// two per wave over every row below (backward). Their gathers are gatherKernel's, before them.
+// wave per 16-row tile of a block; the rows below in 16-row tiles spread over the waves (forward), in
+// batches of 32 rows over every column tile (backward). Their gathers are gatherKernel's, before them.
 
-// Wave-level: a 16-row tile (rows 16·tile within the block) of Inv·Y (TRANSPOSE: Invᵀ·Y) for the unit lower inverse of
-// the diagonal block of qb columns from row q0 (qb × qb column-major at inv), Y the block's rows of ys; the result in
-// the MFMA result layout.
+// A wave's 16-row tile (rows 16·tile within the block) of Inv·Y (TRANSPOSE: Invᵀ·Y) for the unit lower inverse of the
+// diagonal block of qb columns (qb × qb column-major at inv), Y the block's rows of ys from q0: load its operands, times
+// multiplies them, the result in the MFMA result layout.
 template <typename TP> struct InverseTile
 {
     TP a[16];
