@@ -2855,45 +2855,102 @@ __global__ __launch_bounds__(256) void combineValuesKernel(int32_t n, const int6
 // Bound by HBM: a workgroup takes ROW_VALUES_ROWS consecutive rows, whose entries are one range of the CSR, by pieces of
 // ROW_VALUES_PIECE: read and written coalesced through LDS, from which a thread per row sums its entries in their order
 // (a thread per row from memory took 3.1 ms for the 80M entries of the 500 × 500 plate).
-constexpr int ROW_VALUES_ROWS = 128, ROW_VALUES_PIECE = 2048;
+//
+// A piece of long rows holds few of them, and as few threads sum (27 ns an entry): from ROW_VALUES_LONG entries a row
+// on, a piece is the next 16 entries of each of the rows instead, 16 lanes to a row. Setting 6M values, by pieces and by
+// rows: rows of 81 entries 0.105 and 0.107 ms, of 100 0.111 and 0.098, of 300 0.308 and 0.111; a dense matrix of 5,000
+// equations 21.9 and 1.2 ms. A row that is far longer than the others (ROW_VALUES_SPREAD) would leave the lanes of
+// theirs idle for its whole length (2.5 µs per 16 entries, against 56 µs per piece): pieces take it.
+constexpr int ROW_VALUES_ROWS = 128, ROW_VALUES_PIECE = 2048, ROW_VALUES_LONG = 96, ROW_VALUES_SPREAD = 8;
 __global__ __launch_bounds__(256) void rowValuesKernel(int32_t n, const int64_t* csrOffsets, const int64_t* map,
                                                        const double* values, double* csrValues,
                                                        unsigned long long* normKey)
 {
-    __shared__ double piece[ROW_VALUES_PIECE];
+    constexpr int WIDE = 16, PER = ROW_VALUES_PIECE / 256;
+    static_assert(ROW_VALUES_ROWS * WIDE == ROW_VALUES_PIECE, "a piece of long rows");
+    __shared__ double piece[ROW_VALUES_ROWS * (WIDE + 1)];
+    __shared__ int64_t offsets[ROW_VALUES_ROWS + 1], waveLongest[4];
     const int32_t i0 = int32_t(blockIdx.x) * ROW_VALUES_ROWS, i1 = min(i0 + ROW_VALUES_ROWS, n);
     const int32_t i = i0 + int32_t(threadIdx.x);
     const bool owns = threadIdx.x < ROW_VALUES_ROWS && i < i1;
     const int64_t from = csrOffsets[i0], to = csrOffsets[i1];
     const int64_t e0 = owns ? csrOffsets[i] : 0, e1 = owns ? csrOffsets[i + 1] : 0;
     double sum = 0.0;
-    for (int64_t base = from; base < to; base += ROW_VALUES_PIECE)
+    int64_t longest = 0;
+    if (to - from >= int64_t(ROW_VALUES_LONG) * (i1 - i0))
     {
-        const int count = int(min(int64_t(ROW_VALUES_PIECE), to - base));
-        constexpr int PER = ROW_VALUES_PIECE / 256;
-        int64_t at[PER];
-        double v[PER];
-#pragma unroll
-        for (int q = 0; q < PER; ++q)
-            at[q] = map[base + min(int(threadIdx.x) + 256 * q, count - 1)];
-#pragma unroll
-        for (int q = 0; q < PER; ++q)
-            v[q] = values[at[q]];
-#pragma unroll
-        for (int q = 0; q < PER; ++q)
-        {
-            const int e = int(threadIdx.x) + 256 * q;
-            if (e < count)
-            {
-                csrValues[base + e] = v[q];
-                piece[e] = fabs(v[q]);
-            }
-        }
+        if (threadIdx.x <= ROW_VALUES_ROWS)
+            offsets[threadIdx.x] = csrOffsets[min(i, i1)]; // rows beyond the last: empty
+        longest = e1 - e0;
+        for (int offset = 1; offset < 64; offset <<= 1)
+            longest = max(longest, static_cast<int64_t>(__shfl_xor(static_cast<long long>(longest), offset)));
+        if ((threadIdx.x & 63) == 0)
+            waveLongest[threadIdx.x >> 6] = longest;
         __syncthreads();
-        for (int64_t e = max(e0, base); e < min(e1, base + count); ++e)
-            sum += piece[e - base];
-        __syncthreads();
+        for (int w = 0; w < 4; ++w)
+            longest = max(longest, waveLongest[w]);
     }
+    if (longest > 0 && longest * ROW_VALUES_SPREAD <= to - from)
+    {
+        const int lane = int(threadIdx.x) & (WIDE - 1);
+        for (int64_t base = 0; base < longest; base += WIDE)
+        {
+            int64_t at[PER];
+            double v[PER];
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+            {
+                const int r = int(threadIdx.x) / WIDE + 256 / WIDE * q;
+                at[q] = map[min(offsets[r] + base + lane, to - 1)];
+            }
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                v[q] = values[at[q]];
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+            {
+                const int r = int(threadIdx.x) / WIDE + 256 / WIDE * q;
+                const int64_t e = offsets[r] + base + lane;
+                if (e < offsets[r + 1])
+                {
+                    csrValues[e] = v[q];
+                    piece[r * (WIDE + 1) + lane] = fabs(v[q]);
+                }
+            }
+            __syncthreads();
+            const int count = int(min(int64_t(WIDE), e1 - e0 - base));
+            for (int e = 0; e < count; ++e)
+                sum += piece[int(threadIdx.x) * (WIDE + 1) + e];
+            __syncthreads();
+        }
+    }
+    else
+        for (int64_t base = from; base < to; base += ROW_VALUES_PIECE)
+        {
+            const int count = int(min(int64_t(ROW_VALUES_PIECE), to - base));
+            int64_t at[PER];
+            double v[PER];
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                at[q] = map[base + min(int(threadIdx.x) + 256 * q, count - 1)];
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                v[q] = values[at[q]];
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+            {
+                const int e = int(threadIdx.x) + 256 * q;
+                if (e < count)
+                {
+                    csrValues[base + e] = v[q];
+                    piece[e] = fabs(v[q]);
+                }
+            }
+            __syncthreads();
+            for (int64_t e = max(e0, base); e < min(e1, base + count); ++e)
+                sum += piece[e - base];
+            __syncthreads();
+        }
     // Non-negative doubles order as their bit patterns; a row whose sum is not a number is passed over, as the
     // host's std::max passes it over.
     const unsigned long long key = sum == sum ? __double_as_longlong(sum) : 0ull;

@@ -9,8 +9,8 @@ import pytest
 
 import _oracle
 from _problems import block_problem, grid_graph
-from o_o_solver_amd import (BlockSparseMatrix, DeviceMatrix, DofSelection, SparsePattern, SupernodalFactor,
-                            SymmetricCsc, csc_from_blocks_device, models)
+from o_o_solver_amd import (BlockSparseMatrix, DeviceMatrix, DofSelection, FactorSolve, SparsePattern,
+                            SupernodalFactor, SymbolicFactor, SymmetricCsc, csc_from_blocks_device, models)
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +115,38 @@ def test_malformed_block_matrices_are_refused(gpu_device):
     other = DofSelection(np.append(counts, 1))
     with pytest.raises(ValueError, match="was not made for the pattern"):
         csc_from_blocks_device(BlockSparseMatrix(pattern, values), other)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (95, 95), (96, 96), (97, 130, 128, 1), (300,), (2000,) + (3,) * 40, (513, 4),
+                                   (4,) * 31 + (700,), (1500, 1, 1, 1)])
+def test_values_set_on_the_device_equal_those_set_on_the_host(gpu_device, sizes):
+    # Dense blocks along the diagonal: rows around the length from which the row sums are made by rows instead of by
+    # pieces, rows of both kinds in one group of 128, and a last group of few rows. The product reads the rows' copy of
+    # the values, the refined solve's backward error divides by the largest row sum: both to the last bit.
+    import torch
+
+    sizes = np.array(sizes)
+    n, count = int(sizes.sum()), len(sizes)
+    first = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    sym = SymbolicFactor(n, first, sizes, np.full(count, -1), np.zeros(count + 1, np.int64), np.zeros(0, np.int32))
+    lengths = np.concatenate([np.arange(b, 0, -1) for b in sizes])
+    offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    rows = np.arange(offsets[-1]) - np.repeat(offsets[:-1], lengths) + np.repeat(np.arange(n), lengths)
+    rng = np.random.default_rng(n)
+    values = rng.uniform(-1.0, 1.0, offsets[-1])
+    values[offsets[:-1]] = 2.0 * np.repeat(sizes, sizes) * rng.uniform(0.8, 1.2, n)
+    host = SymmetricCsc(n, offsets, rows.astype(np.int32), values)
+    plan = sym.plan()
+    b = torch.from_numpy(rng.standard_normal((2, n))).to("cuda:0").T
+    seen = []
+    for on_device in (False, True):
+        matrix = plan.matrix(SymmetricCsc(n, offsets, host.rows, 3.0 * values))
+        if on_device:
+            matrix.set_values_device(torch.from_numpy(values).to("cuda:0"))
+        else:
+            matrix.set_values(values)
+        factor = SupernodalFactor.factorise(sym, None, device_matrix=matrix)
+        x, report = FactorSolve(factor).solve_refined(b, target=1e-10)
+        seen.append((matrix.multiply(b).cpu().numpy(), x.cpu().numpy(), report.backward_error, factor.diagonal()))
+    for of_host, of_device in zip(*seen):
+        assert np.array_equal(of_host, of_device)
