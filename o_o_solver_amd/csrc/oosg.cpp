@@ -2763,8 +2763,11 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
         // Steps until every front of the level is done, each followed by its trailing update, in rounds: a round
         // launches for each front the steps its candidates need and a few more (a column that interchanges ends its
         // step early), with no wait between them (the launches read the fronts' states on the device, and a front that
-        // is done does nothing), then reads the states. The fronts that need most steps come first, so that every
-        // launch of a round takes the first ones of its list.
+        // is done does nothing), then reads the states. The next round counts on as many columns to a step as the last
+        // one had: fronts whose pivots are mostly 2 × 2 get two a step, and with full panels in every round they took
+        // some thirty rounds with a wait each (a dense matrix of 257 equations with a small diagonal: 2.58 ms, 2.13
+        // now). The fronts that need most steps come first, so that every launch of a round takes the first ones of its
+        // list.
         std::vector<oosg::UpdateTile> tiles;
         std::vector<int32_t> active(count), list32;
         for (int q = 0; q < count; ++q)
@@ -2776,6 +2779,8 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
         for (int q = 0; q < count; ++q)
             maxCand = std::max(maxCand, cand[list[q]]);
         int64_t roundsLeft = 2 * int64_t(maxCand) + 8;
+        std::vector<double> columnsPerStep(static_cast<size_t>(count), 0.0);
+        std::vector<int> stepsTaken(static_cast<size_t>(count), 0);
         while (!active.empty())
         {
             const auto rowsOf = [&](int32_t q) { return pf->order[list[q]] - states[q].k; };
@@ -2788,9 +2793,11 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
             };
             const auto stepsOf = [&](int32_t q)
             {
-                // Panels of half the width where the rows need most registers (eliminatePanel).
-                const int width = oosg::PIVOT_PANEL / (rowsOf(q) > oosg::PIVOT_LARGE_ROWS / 2 ? 2 : 1);
-                const int steps = (cand[list[q]] - states[q].k + width - 1) / width;
+                // A step's columns: the panel's (half the width where the rows need most registers, eliminatePanel), or
+                // those that the front's steps of the last round had.
+                const int panel = oosg::PIVOT_PANEL / (rowsOf(q) > oosg::PIVOT_LARGE_ROWS / 2 ? 2 : 1);
+                const double width = columnsPerStep[q] > 0.0 ? std::min<double>(columnsPerStep[q], panel) : panel;
+                const int steps = static_cast<int>(std::ceil((cand[list[q]] - states[q].k) / width));
                 return steps + steps / 32 + 1;
             };
             std::sort(active.begin(), active.end(),
@@ -2820,7 +2827,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                 for (int J = states[q].k / 64; 64 * J < C; ++J)
                     for (int I = J; 64 * I < N; ++I)
                         trailing.push_back(make_int4(q, I, J, 0));
-                tileSteps.push_back(stepsOf(q));
+                tileSteps.push_back(stepsTaken[q] = stepsOf(q));
                 tileEnd.push_back(static_cast<int>(trailing.size()));
             }
             uploadInto(p.pivotList, list32, st, "factor: active fronts");
@@ -2860,6 +2867,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                     fail(OOSG_INTERNAL, "factor: a front's elimination went back");
                 if (!states[q].done)
                     active[kept++] = q;
+                columnsPerStep[q] = std::max(1.0, static_cast<double>(states[q].k - kBefore[q]) / stepsTaken[q]);
             }
             active.resize(kept);
         }
