@@ -2793,8 +2793,8 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
             };
             const auto stepsOf = [&](int32_t q)
             {
-                // A step's columns: the panel's (half the width where the rows need most registers, eliminatePanel), or
-                // those that the front's steps of the last round had.
+                // A step's columns: the panel's (half of them where the rows need most registers, eliminatePanel, or lie in
+                // memory, pivotColumnsKernel), or those that the front's steps of the last round had.
                 const int panel = oosg::PIVOT_PANEL / (rowsOf(q) > oosg::PIVOT_LARGE_ROWS / 2 ? 2 : 1);
                 const double width = columnsPerStep[q] > 0.0 ? std::min<double>(columnsPerStep[q], panel) : panel;
                 const int steps = static_cast<int>(std::ceil((cand[list[q]] - states[q].k) / width));

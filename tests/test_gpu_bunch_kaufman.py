@@ -142,8 +142,8 @@ def test_weak_children_delay_their_columns_to_the_parent(gpu_device, reference_l
 
 @pytest.mark.parametrize("n,seed", [(3, 1), (40, 2), (130, 3), (257, 4)])
 def test_dense_front_matches_the_oracle_bunch_kaufman(gpu_device, n, seed):
-    # A complete graph is one supernode, its front the whole matrix: the GPU's blocked, left-looking elimination
-    # against the oracle's right-looking one (the reference's order), pivot for pivot.
+    # A complete graph is one supernode, its front the whole matrix: the GPU's elimination by panels against the
+    # oracle's column by column (the reference's order), pivot for pivot.
     graph = clique_graph([list(range(n))], [])
     sym = SymbolicFactor.analyse(graph[0], graph[1], graph[2], np.arange(n, dtype=np.int32))
     assert sym.supernode_count == 1
@@ -225,6 +225,64 @@ def test_tall_fronts_keep_their_inertia(gpu_device, columns, rows):
     full = dense + np.tril(dense, -1).T
     assert np.max(np.abs(full @ x - b)) <= 1e-13 * (np.max(np.sum(np.abs(full), 1)) * np.max(np.abs(x)) +
                                                      np.max(np.abs(b)))
+
+
+def tall_problem(columns, rows, zero):
+    """A supernode of `columns` candidates over `rows` rows and its parent: candidates that interchange and pair among
+    themselves, four that a weak diagonal delays, four that are pivoted alone over a larger row below and, with `zero`,
+    one column of zeros; (symbolic factor, matrix, the supernode's front)."""
+    n = columns + rows
+    sym = SymbolicFactor(n, [0, columns], [columns, rows], [1, -1], [0, rows, rows],
+                         np.arange(columns, n, dtype=np.int32))
+    rng = np.random.default_rng(n)
+    own = np.tril(rng.standard_normal((columns, columns)))
+    own[np.arange(columns), np.arange(columns)] *= rng.choice([1e-3, 1.0, 10.0], columns)
+    below = 1e-3 * rng.standard_normal((rows, columns))
+    special = rng.permutation(columns)[:8]
+    own[special] *= 1e-5
+    own[:, special] *= 1e-5
+    own[special, special] = np.where(np.arange(8) < 4, 1e-5, 0.5)
+    below[:, special] = rng.standard_normal((rows, 8))
+    if zero:
+        at = columns // 2 if columns // 2 not in special else int(np.setdiff1d(np.arange(columns), special)[0])
+        own[at] = own[:, at] = 0.0
+        below[:, at] = 0.0
+    diagonal = 100.0 * np.where(rng.random(rows) < 0.3, -1.0, 1.0)
+    starts = np.concatenate([[0], np.cumsum(np.concatenate([np.arange(n, rows, -1), np.ones(rows, np.int64)]))])
+    index = np.concatenate([np.arange(j, n) for j in range(columns)] + [np.arange(columns, n)]).astype(np.int32)
+    values = np.concatenate([np.concatenate([own[j:, j], below[:, j]]) for j in range(columns)] + [diagonal])
+    front = np.zeros((n, n), order="F")
+    front[:columns, :columns] = own
+    front[columns:, :columns] = below
+    return sym, SymmetricCsc(n, starts.astype(np.int64), index, values), front
+
+
+@pytest.mark.parametrize("columns,rows,zero", [(40, 2100, True), (60, 2020, False), (50, 4040, False), (45, 4200, False),
+                                               (40, 4200, True)])
+def test_tall_fronts_match_the_oracle_bunch_kaufman(gpu_device, columns, rows, zero):
+    # Every branch of the pivot tests where a thread holds eight rows of eight columns (2,049 to 4,096 rows; from 2,048
+    # rows on, four rows of sixteen) and where the columns go through memory (more): the oracle's pivots exactly.
+    # Values: the growth of the multipliers (4/0.5 and 1/0.36 a column) over a few columns, times eps, is below 1e-9.
+    sym, m, front = tall_problem(columns, rows, zero)
+    n = columns + rows
+    perm, sub = np.zeros(columns, np.int64), np.zeros(columns)
+    e = _oracle.oracle().orc_bunch_kaufman(_oracle.P(front), n, n, columns, _oracle.P(perm), _oracle.P(sub))
+    pivots = np.diag(front)[:e]
+    assert columns - e == 4 and np.count_nonzero(sub[:e]) >= 4 and np.count_nonzero(pivots == 0.0) == int(zero)
+    assert not np.array_equal(perm, np.arange(columns))
+    f = SupernodalFactor.factorise(sym, m, INDEFINITE)
+    values, index = f.panel(0)
+    assert f.delayed_pivot_count == columns - e and values.shape == (n, e)
+    assert index.tolist() == perm.tolist() + list(range(columns, n))
+    assert np.allclose(f.subdiagonal(0), sub[:e], rtol=1e-9, atol=0)
+    lower = np.tril(front[:, :e], -1)
+    assert np.max(np.abs(np.tril(values, -1) - lower)) <= 1e-9 * max(1.0, np.max(np.abs(lower)))
+    assert np.max(np.abs(np.diag(values) - pivots)) <= 1e-9 * np.max(np.abs(pivots))
+    assert f.inertia.zero == int(zero)
+    if not zero:
+        b = np.random.default_rng(rows).standard_normal((n, 2))
+        x = FactorSolve(f).solve(b)
+        assert backward_error(m, x, b) <= 1e-12
 
 
 @pytest.mark.parametrize("sizes,seed", [((5, 7, 6), 1), ((70, 90, 40), 3), ((300, 420, 200), 5)])
