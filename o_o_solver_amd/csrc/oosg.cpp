@@ -447,9 +447,9 @@ struct oosg_plan
         double flops[2] = {0.0, 0.0};
     };
     std::vector<int4> inverseItems;
-    // By level, for the streams beside the critical path; and all levels' together, for one stream after the last
-    // level (a round per height of the halvings: the first product's launch, then the second's).
-    std::vector<std::vector<InverseRound>> inverseRounds;
+    // All levels' together, for one stream after the last level (a round per height of the halvings: the first
+    // product's launch, then the second's). The schedule has them by level beside that, for the streams beside the
+    // critical path.
     std::vector<InverseRound> mergedInverses;
     int32_t levels = 0;
     int64_t smallFronts = 0, largeFronts = 0;
@@ -1162,7 +1162,7 @@ void addDiagonalInverseItems(oosg_plan& p, int32_t s)
 }
 
 // The rounds of a level's whole inverses for a stream beside the critical path: at every INVERSE_BLOCKS column blocks
-// whose panel solve is done, and at the level's end, the products whose operands are there, round by round.
+// whose panel solve is done, and at the level's end (maxBlocks), the products whose operands are there, round by round.
 std::vector<oosg_plan::InverseRound> levelInverseRounds(oosg_plan& p, int32_t l, int maxBlocks)
 {
     std::vector<oosg_plan::InverseRound> rounds;
@@ -1352,14 +1352,11 @@ void deriveLevels(oosg_plan& p)
         fail(OOSG_INVALID_ARGUMENT, "plan: more than 2^31 rows below the supernodes");
     for (int32_t l = 0; l < p.levels; ++l)
     {
-        int maxBlocks = 0;
         int32_t forwardSlots = 0, backwardSlots = 0; // each sweep's slots of this level
         for (int32_t q = p.levelStart[l]; q < p.levelStart[l + 1]; ++q)
         {
             const int32_t s = p.levelList[q];
             const bool wide = p.ncol[s] >= oosg::WIDE_COLUMNS;
-            if (wide)
-                maxBlocks = std::max(maxBlocks, (p.ncol[s] + 63) / 64);
             // The L_RF products of every supernode with rows below but the small ones (those do them in the
             // workgroup of their triangle): row tiles (forward), column blocks (backward). A supernode of a pivoted
             // factor whose columns were all delayed has none (c = 0).
@@ -1436,7 +1433,6 @@ void deriveLevels(oosg_plan& p)
         p.forwardTriangleStart[l + 1] = static_cast<int64_t>(p.forwardTriangles.size());
         p.backwardTriangleStart[l + 1] = static_cast<int64_t>(p.backwardTriangles.size());
         p.triangleSumStart[l + 1] = static_cast<int64_t>(p.forwardTriangleSums.size());
-        p.inverseRounds.push_back(levelInverseRounds(p, l, maxBlocks));
     }
     mergeInverses(p);
     placeUpdateMatrices(p, height);
@@ -1659,6 +1655,7 @@ void buildSchedule(oosg_plan& p)
             }
         }
         p.schedule.push_back(assemble);
+        const std::vector<oosg_plan::InverseRound> inverseRounds = levelInverseRounds(p, l, (maxC + 63) / 64);
         // Panel steps.
         // A record of EVENT_SOLVED on the critical stream delays its next launch by several microseconds, so a step
         // records only when the bulk update or a round of the whole inverses needs it, and at the level's last step.
@@ -1789,7 +1786,7 @@ void buildSchedule(oosg_plan& p)
             // The whole inverses' rounds whose panels this step completes run beside the next steps.
             const int solvedBlocks = k0 / PANEL_BLOCK + 1;
             bool waits = true;
-            for (const oosg_plan::InverseRound& round : p.inverseRounds[l])
+            for (const oosg_plan::InverseRound& round : inverseRounds)
                 if (round.ready == solvedBlocks && solvedBlocks % INVERSE_BLOCKS == 0 && k0 + PANEL_BLOCK < maxC)
                 {
                     pushInverseRound(p, round, waits ? EVENT_SOLVED : -1);
@@ -1875,7 +1872,7 @@ void buildSchedule(oosg_plan& p)
         }
         // The rest of the level's whole inverses, once its panels are final.
         bool waits = true;
-        for (const oosg_plan::InverseRound& round : p.inverseRounds[l])
+        for (const oosg_plan::InverseRound& round : inverseRounds)
             if (round.ready % INVERSE_BLOCKS != 0 || round.ready * PANEL_BLOCK >= maxC)
             {
                 pushInverseRound(p, round, waits ? EVENT_PANELS : -1);
