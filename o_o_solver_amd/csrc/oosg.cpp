@@ -761,8 +761,11 @@ void pollCancellation(oosg_plan& p)
 
 // ---- plan --------------------------------------------------------------------------------------------------------
 
-// The column blocks solved between two rounds of the whole inverses beside a level's panel steps.
-constexpr int INVERSE_BLOCKS = 8;
+// The column blocks solved between two rounds of the whole inverses beside a level's panel steps. In a graph of three
+// streams a round costs its dependencies: the 24³ hex block's factorisation took 7.07, 6.61 and 6.26 ms with rounds every
+// 4, 8 and 16 blocks, the 500 × 500 plate's 34.5, 33.6 and 32.9 ms; launched one at a time the spacing makes no
+// difference (5.72, 5.76 and 5.79 ms; 31.4, 31.3 and 31.2 ms).
+constexpr int INVERSE_BLOCKS = 16;
 
 void deriveLevels(oosg_plan& p);
 oosg_status createPlan(const oosg_symbolic_desc* symbolic, int32_t trailing_dof_count, bool outOfCore, int32_t device,

@@ -48,3 +48,36 @@ def test_panels_match_the_dense_factor(gpu_device, c, r, precision):
     b = np.random.default_rng(7).standard_normal((c + r, 3))
     x = FactorSolve(factor).solve(b)
     assert np.max(np.abs(x - np.linalg.solve(dense, b))) <= tolerance * np.max(np.abs(x))
+
+
+@pytest.mark.parametrize("precision", [Precision.FP64, Precision.FP32])
+@pytest.mark.parametrize("widths", [(1025,), (576, 1090), (1024, 512, 200), (40, 2113)])
+def test_inverses_beside_the_panel_steps_give_the_same_bits(gpu_device, widths, precision):
+    # Supernodes of one level over a common parent: on three streams the whole inverses of those with more than sixteen
+    # blocks of 64 columns follow every sixteen blocks beside the panel steps, on one stream all levels' come last. The
+    # products and their order are the same, so are the panels and (through the inverses) the solutions.
+    rows = 40
+    children = len(widths)
+    n = sum(widths) + rows
+    first = np.concatenate([[0], np.cumsum(widths)])
+    sym = SymbolicFactor(n, first, list(widths) + [rows], [children] * children + [-1],
+                         rows * np.minimum(np.arange(children + 2), children),
+                         np.tile(np.arange(n - rows, n, dtype=np.int32), children))
+    rng = np.random.default_rng(n)
+    index = [np.concatenate([np.arange(j, first[s] + c), np.arange(n - rows, n)]) for s, c in enumerate(widths)
+             for j in range(first[s], first[s] + c)] + [np.arange(j, n) for j in range(n - rows, n)]
+    offsets = np.concatenate([[0], np.cumsum([i.size for i in index])]).astype(np.int64)
+    values = rng.uniform(-1.0, 1.0, offsets[-1])
+    values[offsets[:-1]] = 2.0 * n * rng.uniform(0.8, 1.2, n)
+    plan = sym.plan()
+    matrix = plan.matrix(SymmetricCsc(n, offsets, np.concatenate(index).astype(np.int32), values))
+    options = FactorOptions(precision=precision)
+    b = rng.standard_normal((n, 3))
+    expected = None
+    for mode in ("graph", "eager_streams", "graph_streams", "eager_streams"):
+        plan.launch_mode(precision, mode)
+        factor = SupernodalFactor.factorise(sym, None, options, device_matrix=matrix)
+        got = [factor.panel(s)[0] for s in range(children + 1)] + [FactorSolve(factor).solve(b)]
+        del factor
+        expected = expected or got
+        assert all(np.array_equal(x, y) for x, y in zip(got, expected)), mode
