@@ -483,6 +483,32 @@ def test_ratio_test_statistics_match_the_pivots(gpu_device, precision):
         assert abs(g.pivot_diagnostics.largest_ratio - np.max(oracle_ratio)) <= 1e-9 * np.max(oracle_ratio)
 
 
+def test_issues_name_the_diagonal_of_the_values_in_force(gpu_device):
+    # The matrix diagonal that an issue (or the bail-out's message) names is that of the values last set, on whichever
+    # side they were set: it is read from the device when first needed.
+    import torch
+    w = CASES["plate 12"]()
+    sym = w.analyse()
+    m = w.matrix
+    plan = sym.plan()
+    dm, k = plan.matrix(m), plan.matrix(m)
+    options = FactorOptions(pivot_policy=oos.PivotPolicy(max_ratio=1.5, bailout=-1))
+    diagonal = m.values[m.offsets[:-1]]
+
+    def named(factor):
+        issues = SupernodalFactor.factorise(sym, None, options, device_matrix=dm).pivot_diagnostics.issues
+        assert len(issues) > 10
+        return all(i.matrix_diagonal == factor * diagonal[i.equation] for i in issues)
+
+    assert named(1.0)
+    dm.set_values_device(torch.from_numpy(2.0 * m.values).to("cuda:0"))
+    assert named(2.0) and named(2.0)
+    dm.set_combination(3.0, k, 1.0, k)
+    assert named(4.0)
+    dm.set_values(8.0 * m.values)
+    assert named(8.0)
+
+
 @pytest.mark.parametrize("precision", [Precision.FP64, Precision.FP32])
 def test_factorise_and_solve_equals_the_two_calls(gpu_device, precision):
     # The combined call sweeps the lower levels forward beside the factorisation of the top ones (in the eager
