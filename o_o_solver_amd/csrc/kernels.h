@@ -223,7 +223,8 @@ hipError_t launchExtendTiles(const DevicePlan& p, T* panels, T* updates, const U
 template <typename T>
 hipError_t launchUpdateTiles(const DevicePlan& p, T* panels, T* updates, T* linv, const UpdateTile* tiles, int count,
                              double* diagOut, int32_t* zeroAt, bool fused, hipStream_t stream);
-// One level of the forward sweep: the supernodes of `list` (gathered, below WIDE_COLUMNS columns), then the row tiles (supernode, tile) of its big ones.
+// One level of the forward sweep: the supernodes of `list` (gathered, below WIDE_COLUMNS columns), then the row tiles
+// (supernode, tile) of its big ones.
 template <typename TP>
 hipError_t launchForward(const DevicePlan& p, const TP* panels, const TP* linv, double* X, double* U, int k,
                          const int32_t* list, int count, const int4* rowTiles, int tileCount, double* partials,

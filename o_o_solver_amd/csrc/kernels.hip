@@ -305,9 +305,9 @@ __global__ __launch_bounds__(256) void smallFrontKernel(DevicePlan p, DeviceMatr
 
 // Assembly of a block of a front: columns [j0, j1), rows [i0, i1), accumulated in LDS in the reference's order (zero,
 // the matrix entries, the children in increasing order), then its lower part written to the panel (columns < c; the
-// panel's values above the diagonal are never read, nor written) or to the update matrix. The matrix entries of the block's columns are one range
-// of the CSC, spread over the threads; a child's part, its columns by consecutive rows, too, so that every thread has
-// several independent loads in flight whatever the block's shape.
+// panel's values above the diagonal are not assembled: nothing reads them) or to the update matrix. The matrix entries of
+// the block's columns are one range of the CSC, spread over the threads; a child's part, its columns by consecutive rows,
+// too, so that every thread has several independent loads in flight whatever the block's shape.
 template <typename T>
 __global__ __launch_bounds__(256) void assembleKernel(DevicePlan p, DeviceMatrix a, T* panels, T* updates,
                                                       const AssemblyBlock* blocks, const AssemblyItem* items)

@@ -1126,8 +1126,6 @@ void windowLayout(oosg_plan& p, const std::vector<int32_t>& height)
     p.linvOff[S] = 2 * p.windowLinv;
 }
 
-// From the structure (first, ncol, nrow, parent, children): the offsets of the panels, update matrices and inverses,
-// the levels by height, the flops, and the sweeps' work lists by level.
 // The halvings of a wide triangle's column blocks: node [a, b) with its middle, the nodes of its halves (-1: a single
 // block, whose inverse the factorisation gives) and its height. Children come before their parents.
 struct Halving
@@ -1258,6 +1256,8 @@ void mergeInverses(oosg_plan& p)
     }
 }
 
+// From the structure (first, ncol, nrow, parent, children): the offsets of the panels, update matrices and inverses,
+// the levels by height, the flops, the sweeps' work lists by level and the whole inverses' rounds of all levels.
 void deriveLevels(oosg_plan& p)
 {
     const int32_t S = p.S;
@@ -1462,9 +1462,7 @@ Launch syncLaunch(int lane, int wait, int record)
     return l;
 }
 
-// A launch of one step of a level's whole inverses, on the inverses' stream after the event `wait`.
-// The launch of a step's row block finals (before the step's own launch).
-// The launches of a round of the whole inverses, the first after `wait`.
+// The launches of a round of the whole inverses, on the inverses' stream, the first after the event `wait`.
 void pushInverseRound(oosg_plan& p, const oosg_plan::InverseRound& round, int wait)
 {
     for (int which = 0; which < 2; ++which)
@@ -1964,7 +1962,8 @@ void uploadPlan(oosg_plan& p)
 // The plan's own arrays on the device (structure, launch lists), in bytes.
 uint64_t structureBytes(const oosg_plan& p)
 {
-    return (p.first.size() * 3 + p.rows.size() * 2 + p.children.size() + p.smallList.size() + p.levelList.size() * 2 + p.mediumList.size() + p.pullBase.size() + p.pulls.size() + p.gatherStart.size() +
+    return (p.first.size() * 3 + p.rows.size() * 2 + p.children.size() + p.smallList.size() +
+            p.levelList.size() * 2 + p.mediumList.size() + p.pullBase.size() + p.pulls.size() + p.gatherStart.size() +
             p.gatherRows.size() + p.otherPosStart.size() * 2 + p.gatherChunks.size() * 8) *
                4 +
            p.panelOff.size() * 24 +
@@ -1972,7 +1971,8 @@ uint64_t structureBytes(const oosg_plan& p)
             p.backwardSubtractions.size()) *
                16 +
            (p.forwardTriangles.size() + p.backwardTriangles.size() + 2 * p.forwardTriangleSums.size()) * 16 +
-           p.inverseItems.size() * 16 + p.diagonalBlocks.size() * sizeof(oosg::DiagonalBlock) + p.blocks.size() * sizeof(oosg::AssemblyBlock) +
+           p.inverseItems.size() * 16 + p.diagonalBlocks.size() * sizeof(oosg::DiagonalBlock) +
+           p.blocks.size() * sizeof(oosg::AssemblyBlock) +
            p.items.size() * sizeof(oosg::AssemblyItem) +
            (p.tiles.size() + p.bigTiles.size()) * sizeof(oosg::UpdateTile) + p.itemStarts.size() * 4 +
            p.extendItems.size() * sizeof(oosg::AssemblyItem) +
@@ -2627,11 +2627,11 @@ void permuteSweepPlan(const oosg_plan& p, oosg_plan& d, const PivotedFactor& pf,
 
 // The indefinite factorisation (MultifrontalDriver::eliminatePivoted, MultifrontalDriver.cpp:346-436), level by level:
 // each front [own columns, the columns its children delayed (in child order), rows] is assembled, eliminated with
-// Bunch–Kaufman pivoting among its candidates in blocks of PANEL_BLOCK columns, the candidates it cannot eliminate
-// delayed to its parent; a root front cannot delay. The host reads each front's state after every block step (the
-// trailing tiles depend on how far it got) and its permutation after the level. Then the panels (the first e columns
-// of each front) are packed, the structure in pivot order is built for the sweeps, and the inverses of the unit
-// lower triangles are formed.
+// Bunch–Kaufman pivoting among its candidates in steps of up to PIVOT_PANEL columns, the candidates it cannot eliminate
+// delayed to its parent; a root front cannot delay. The steps go in rounds without a wait between them; the host reads
+// each front's state after a round and its permutation after the level. Then the panels (the first e columns of each
+// front) are packed, the structure in pivot order is made for the sweeps (the plan's own lists where no column was
+// delayed), and the inverses of the unit lower triangles are formed.
 void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
 {
     const hipStream_t st = p.stream;
@@ -5584,8 +5584,8 @@ oosg_status oosg_factor_panel(const oosg_factor* f, int32_t s, double* values, i
                 check(hipMemcpy(values, f->panels.as<double>() + p.panelOff[s], count * sizeof(double),
                                 hipMemcpyDeviceToHost),
                       "panel: copy");
-            // The device never reads or writes the values above the diagonal (their memory may hold other values, an
-            // out-of-core window another level's): they are zeros here, as in the reference's panels.
+            // The device never reads the values above the diagonal (full diagonal blocks hold their inverse's transpose
+            // there, an out-of-core window another level's values): they are zeros here, as in the reference's panels.
             const int64_t n = c + r;
             for (int64_t j = 1; j < c; ++j)
                 std::fill(values + j * n, values + j * n + j, 0.0);
