@@ -33,7 +33,7 @@ METRIC = "factor+solve s at 1e-10 backward err: mixed FP32+IR vs FP64 GPU; % MFM
 PEAK_FP64 = 78.6   # TFLOP/s, MI355X dense FP64 matrix
 PEAK_FP32 = 157.3  # TFLOP/s, MI355X dense FP32 matrix
 PEAK_HBM = 8000.0  # GB/s, MI355X HBM3E
-# The HIP kernel behind each profile kind, as a rocprofv3 trace names it ({T}: double or float).
+# The HIP kernel behind each profile kind, as a rocprofv3 trace names it ({T}: double or float; *: any).
 KIND_KERNELS = {"small_fronts": "smallFrontKernel<{T}>", "assembly": "assembleKernel<{T}>",
                 "diagonal_blocks": "diagonalBlockKernel<{T}>",
                 "panel_solve": "updateTilesKernel<{T},false,false>",
@@ -44,7 +44,7 @@ KIND_KERNELS = {"small_fronts": "smallFrontKernel<{T}>", "assembly": "assembleKe
                 "forward_triangles": "forwardKernel<{T}>", "backward_triangles": "backwardKernel<{T}>",
                 "residual": "multiplyRowsKernel", "forward_rows": "forwardRowsKernel<{T}>",
                 "backward_columns": "backwardColumnsKernel<{T}>", "triangle_products": "triangleProductsKernel<{T}>",
-                "triangle_inverses": "triangleInverseKernel<{T}>"}
+                "triangle_inverses": "triangleInverseKernel<{T},*>"}  # its two products
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "hbm_traffic_shell_plate_c2.txt")
 BYTE_KINDS = ("assembly", "forward_triangles", "backward_triangles", "residual", "forward_rows", "backward_columns",
               "triangle_products")

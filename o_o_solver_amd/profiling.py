@@ -26,6 +26,7 @@ read_traffic(path, kernel) returns the calibrated bytes per launch of one kernel
 import argparse
 import csv
 import collections
+import fnmatch
 import os
 import re
 import sys
@@ -151,17 +152,20 @@ def mfma(csv_path, out, command, stats_path=None):
 
 
 def read_traffic(path, kernel):
-    """The calibrated HBM bytes per launch of `kernel` in a traffic summary, or None."""
+    """The calibrated HBM bytes per launch of `kernel` (with `*`: of every kernel of that form) in a traffic summary, or
+    None."""
     if not os.path.exists(path):
         return None
+    launches, total = 0, 0.0
     with open(path) as f:
         for line in f:
             if line.startswith("#"):
                 continue
             parts = line.split()
-            if len(parts) == 5 and parts[0] == kernel:
-                return float(parts[4])
-    return None
+            if len(parts) == 5 and fnmatch.fnmatchcase(parts[0], kernel):
+                launches += int(parts[1])
+                total += int(parts[1]) * float(parts[4])
+    return total / launches if launches else None
 
 
 def factorisations(csv_path):
