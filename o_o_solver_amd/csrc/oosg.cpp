@@ -2765,9 +2765,12 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
         // step early), with no wait between them (the launches read the fronts' states on the device, and a front that
         // is done does nothing), then reads the states. The next round counts on as many columns to a step as the last
         // one had: fronts whose pivots are mostly 2 × 2 get two a step, and with full panels in every round they took
-        // some thirty rounds with a wait each (a dense matrix of 257 equations with a small diagonal: 2.58 ms, 2.13
-        // now). The fronts that need most steps come first, so that every launch of a round takes the first ones of its
-        // list.
+        // some thirty rounds with a wait each (a dense matrix of 257 equations with a small diagonal: 2.55 ms, 2.15
+        // now). What is launched for nothing stays below what the fronts need: no round has more than twice the steps of
+        // the last one, and a front that delays columns keeps counting on full panels, as most of what it has left may
+        // stay delayed (16 plates of random values, 117 columns delayed and 18,894 pairs: 58 ms with full panels, 61 with
+        // each front's own rate, 57.5 now; with random diagonals and 69,000 columns delayed 194, 198 and 194 ms). The
+        // fronts that need most steps come first, so that every launch of a round takes the first ones of its list.
         std::vector<oosg::UpdateTile> tiles;
         std::vector<int32_t> active(count), list32;
         for (int q = 0; q < count; ++q)
@@ -2779,7 +2782,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
         for (int q = 0; q < count; ++q)
             maxCand = std::max(maxCand, cand[list[q]]);
         int64_t roundsLeft = 2 * int64_t(maxCand) + 8;
-        std::vector<double> columnsPerStep(static_cast<size_t>(count), 0.0);
+        double columnsPerStep = 0.0; // of the last round's fronts that go on and delay nothing (0: none)
         std::vector<int> stepsTaken(static_cast<size_t>(count), 0);
         while (!active.empty())
         {
@@ -2791,21 +2794,24 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                        : rows <= oosg::PIVOT_LARGE_ROWS ? oosg::PIVOT_LARGE
                                                         : oosg::PIVOT_ANY;
             };
+            const auto delays = [&](int32_t q)
+            { return states[q].end < cand[list[q]] || states[q].passStart > 0; };
             const auto stepsOf = [&](int32_t q)
             {
                 // A step's columns: the panel's (half of them where the rows need most registers, eliminatePanel, or lie in
-                // memory, pivotColumnsKernel), or those that the front's steps of the last round had.
+                // memory, pivotColumnsKernel), or those that a step of the last round had.
                 const int panel = oosg::PIVOT_PANEL / (rowsOf(q) > oosg::PIVOT_LARGE_ROWS / 2 ? 2 : 1);
-                const double width = columnsPerStep[q] > 0.0 ? std::min<double>(columnsPerStep[q], panel) : panel;
-                const int steps = static_cast<int>(std::ceil((cand[list[q]] - states[q].k) / width));
+                const double width = columnsPerStep > 0.0 && !delays(q) ? std::min<double>(columnsPerStep, panel) : panel;
+                int steps = static_cast<int>(std::ceil((cand[list[q]] - states[q].k) / width));
+                if (stepsTaken[q] > 0)
+                    steps = std::min(steps, 2 * stepsTaken[q]);
                 return steps + steps / 32 + 1;
             };
+            for (const int32_t q : active)
+                stepsTaken[q] = stepsOf(q);
             std::sort(active.begin(), active.end(),
                       [&](int32_t x, int32_t y)
-                      {
-                          const int sx = stepsOf(x), sy = stepsOf(y);
-                          return sx != sy ? sx > sy : x < y;
-                      });
+                      { return stepsTaken[x] != stepsTaken[y] ? stepsTaken[x] > stepsTaken[y] : x < y; });
             list32.clear();
             trailing.clear();
             std::vector<int> kindStart(oosg::PIVOT_KINDS + 1, 0);
@@ -2816,7 +2822,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                     if (kindOf(q) == kind)
                     {
                         list32.push_back(q);
-                        kindSteps[kind].push_back(stepsOf(q));
+                        kindSteps[kind].push_back(stepsTaken[q]);
                     }
                 kindStart[kind + 1] = static_cast<int>(list32.size());
             }
@@ -2827,7 +2833,7 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                 for (int J = states[q].k / 64; 64 * J < C; ++J)
                     for (int I = J; 64 * I < N; ++I)
                         trailing.push_back(make_int4(q, I, J, 0));
-                tileSteps.push_back(stepsTaken[q] = stepsOf(q));
+                tileSteps.push_back(stepsTaken[q]);
                 tileEnd.push_back(static_cast<int>(trailing.size()));
             }
             uploadInto(p.pivotList, list32, st, "factor: active fronts");
@@ -2861,15 +2867,21 @@ void factorisePivoted(oosg_plan& p, const oosg_matrix& m, oosg_factor& f)
                   "factor: front states");
             check(hipStreamSynchronize(st), "factor: Bunch-Kaufman");
             size_t kept = 0;
+            double columns = 0.0, stepsOfRound = 0.0;
             for (const int32_t q : active)
             {
                 if (states[q].k < kBefore[q] || states[q].k > cand[list[q]])
                     fail(OOSG_INTERNAL, "factor: a front's elimination went back");
                 if (!states[q].done)
                     active[kept++] = q;
-                columnsPerStep[q] = std::max(1.0, static_cast<double>(states[q].k - kBefore[q]) / stepsTaken[q]);
+                if (!states[q].done && !delays(q))
+                {
+                    columns += states[q].k - kBefore[q];
+                    stepsOfRound += stepsTaken[q];
+                }
             }
             active.resize(kept);
+            columnsPerStep = stepsOfRound > 0.0 ? std::max(1.0, columns / stepsOfRound) : 0.0;
         }
         // The rows below the candidates: their update matrix part −= L·Wᵀ over the eliminated columns.
         tiles.clear();
